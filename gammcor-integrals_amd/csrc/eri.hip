@@ -699,17 +699,7 @@ void eri_run(Context &C, const EriRequest &R) {
   // per-class statistics time every launch on its own, so they stay on the
   // context stream; otherwise the launches are spread over the side streams
   const int nstream = stats ? 1 : (int)std::min<long long>(C.eri_streams, (long long)prep.size());
-  if (nstream > 1) {
-    if (!C.eri_fork) {
-      GI_HIP(hipEventCreateWithFlags(&C.eri_fork, hipEventDisableTiming));
-      for (int j = 0; j < Context::ERI_MAX_STREAMS - 1; ++j) {
-        GI_HIP(hipStreamCreateWithFlags(&C.eri_side[j], hipStreamNonBlocking));
-        GI_HIP(hipEventCreateWithFlags(&C.eri_join[j], hipEventDisableTiming));
-      }
-    }
-    GI_HIP(hipEventRecord(C.eri_fork, C.stream));
-    for (int j = 1; j < nstream; ++j) GI_HIP(hipStreamWaitEvent(C.eri_side[j - 1], C.eri_fork, 0));
-  }
+  C.fork_side(nstream);
   std::vector<size_t> order(prep.size());
   for (size_t i = 0; i < order.size(); ++i) order[i] = i;
   std::stable_sort(order.begin(), order.end(), [&](size_t x, size_t y) { return prep[x].fl > prep[y].fl; });
@@ -748,10 +738,7 @@ void eri_run(Context &C, const EriRequest &R) {
       (void)hipEventDestroy(s1);
     }
   }
-  for (int j = 1; j < nstream; ++j) {
-    GI_HIP(hipEventRecord(C.eri_join[j - 1], C.eri_side[j - 1]));
-    GI_HIP(hipStreamWaitEvent(C.stream, C.eri_join[j - 1], 0));
-  }
+  C.join_side(nstream);
   if (C.time_eri) {
     GI_HIP(hipEventRecord(e1, C.stream));
     GI_HIP(hipEventSynchronize(e1));

@@ -50,6 +50,7 @@ Context::~Context() {
   chol.mo_adj_p.release();
   release_chol_work(*this);
   release_thc_work(*this);
+  release_grad_work(*this);
   for (int i = 0; i < 2; ++i) {
     spl_slices[i].release();
     spl_exp[i].release();
@@ -78,6 +79,26 @@ void Context::wait() {
     GI_HIP(hipEventSynchronize(wait_ev));
   }
   xfer_used = 0;   // every staged copy has completed
+}
+
+void Context::fork_side(int n) {
+  if (n <= 1) return;
+  if (!eri_fork) {
+    GI_HIP(hipEventCreateWithFlags(&eri_fork, hipEventDisableTiming));
+    for (int j = 0; j < ERI_MAX_STREAMS - 1; ++j) {
+      GI_HIP(hipStreamCreateWithFlags(&eri_side[j], hipStreamNonBlocking));
+      GI_HIP(hipEventCreateWithFlags(&eri_join[j], hipEventDisableTiming));
+    }
+  }
+  GI_HIP(hipEventRecord(eri_fork, stream));
+  for (int j = 1; j < n; ++j) GI_HIP(hipStreamWaitEvent(eri_side[j - 1], eri_fork, 0));
+}
+
+void Context::join_side(int n) {
+  for (int j = 1; j < n; ++j) {
+    GI_HIP(hipEventRecord(eri_join[j - 1], eri_side[j - 1]));
+    GI_HIP(hipStreamWaitEvent(stream, eri_join[j - 1], 0));
+  }
 }
 
 unsigned char *Context::xfer_slot(size_t bytes) {

@@ -89,6 +89,7 @@ struct CholState {
 
 struct CholWork;   // gi_chol_build work arrays (chol.hip)
 struct ThcWork;    // work arrays of the THC calls (thc.hip)
+struct GradWork;   // work arrays of the Coulomb energy and gradient (grad.hip)
 
 struct Context {
   int device = 0;
@@ -136,6 +137,8 @@ struct Context {
   CholWork *cw = nullptr;
   // device work arrays of the THC calls (thc.hip), grow-only
   ThcWork *thcw = nullptr;
+  // device work arrays of the Coulomb energy and gradient (grad.hip), grow-only
+  GradWork *gradw = nullptr;
   // split-BF16 products (split.hip): BF16 slice planes and per-chunk row
   // scale exponents of the two operands; grow-only, kept across calls
   DBuf<unsigned short> spl_slices[2];
@@ -197,6 +200,10 @@ struct Context {
   long long eri_streams = ERI_MAX_STREAMS;
   hipStream_t eri_side[ERI_MAX_STREAMS - 1] = {};
   hipEvent_t eri_fork = nullptr, eri_join[ERI_MAX_STREAMS - 1] = {};
+  // fork_side: streams 1..n-1 (eri_side) wait for the work on the context
+  // stream; join_side: the context stream waits for them
+  void fork_side(int n);
+  void join_side(int n);
 
   Context(int dev);
   ~Context();
@@ -251,6 +258,12 @@ long long chol_factor_inverse_scratch(long long n);
 // one md_kernel<E, F> launch (eri.hip)
 void launch_md_class(int E, int F, const MdArgs &a, int grid, hipStream_t s);
 
+// Hermite Coulomb potentials on primitive pairs (coul_kernel.h): class
+// kernels for bra order E <= COUL_EMAX and ket order F <= COUL_FMAX
+struct CoulArgs;
+struct CoulKet;
+void launch_coul_j(int E, int F, const CoulArgs &a, int groups, hipStream_t s);
+
 // density-contracted pair tables of the Coulomb gradient (grad_kernels.h, eri.hip)
 constexpr int GRAD_NCOL = 10;   // columns per primitive pair table
 struct GradJob {
@@ -281,6 +294,7 @@ void thc_rkab(Context &C, const double *dX, long long ldx, long long npts, const
 void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_thresh, double qr_thresh_reduced,
                      long long block_dim, std::vector<long long> &pivots, long long &nred);
 void release_thc_work(Context &C);
+void release_grad_work(Context &C);
 
 // Coulomb energy of a density and its nuclear gradient (grad.hip)
 void coulomb_energy_grad(Context &C, const double *D, long long ldd, double kappa, double *energy,

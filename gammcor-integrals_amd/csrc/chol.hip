@@ -195,36 +195,31 @@ __global__ void k_gather_block(double *__restrict__ Mb, const double *__restrict
   if (e < nb && c < nb) Mb[e + nb * c] = M[bd[e] + ldM * c];
 }
 
-// first maximum over a 1024-lane workgroup (key descending, index ascending;
-// the order of merging does not change the result).  Ends with a barrier.
-__device__ void wg_argmax_1024(double &k, double &v, int &i) {
-  __shared__ double sk[16], sv[16];
-  __shared__ int si[16];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const double k2 = __shfl_xor(k, off), v2 = __shfl_xor(v, off);
-    const int i2 = __shfl_xor(i, off);
-    const bool take = (i2 >= 0) && (i < 0 || k2 > k || (k2 == k && i2 < i));
-    if (take) { k = k2; v = v2; i = i2; }
-  }
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0) { sk[w] = k; sv[w] = v; si[w] = i; }
-  __syncthreads();
-  if (w == 0) {
-    if (lane < 16) { k = sk[lane]; v = sv[lane]; i = si[lane]; }
-    else { i = -1; }
-#pragma unroll
-    for (int off = 8; off > 0; off >>= 1) {
-      const double k2 = __shfl_xor(k, off), v2 = __shfl_xor(v, off);
-      const int i2 = __shfl_xor(i, off);
-      const bool take = (i2 >= 0) && (i < 0 || k2 > k || (k2 == k && i2 < i));
-      if (take) { k = k2; v = v2; i = i2; }
-    }
-    if (lane == 0) { sk[0] = k; sv[0] = v; si[0] = i; }
-  }
-  __syncthreads();
-  k = sk[0]; v = sv[0]; i = si[0];
-  __syncthreads();
+// maximum over the wavefront (NaN ignored), the same value in every lane: the
+// rows of sixteen by row shifts, then the row totals by row broadcasts, lane 63
+// last
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_max(double x) {
+  const unsigned long long v = __builtin_bit_cast(unsigned long long, x);
+  const int lo = __builtin_amdgcn_update_dpp((int)v, (int)v, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp((int)(v >> 32), (int)(v >> 32), CTRL, ROWS, 0xf, false);
+  return fmax(x, __builtin_bit_cast(double, (unsigned long long)(unsigned)lo | ((unsigned long long)(unsigned)hi << 32)));
+}
+__device__ __forceinline__ double wave_max(double x) {
+  x = dpp_max<0x111, 0xf>(x);   // row_shr:1, 2, 4, 8
+  x = dpp_max<0x112, 0xf>(x);
+  x = dpp_max<0x114, 0xf>(x);
+  x = dpp_max<0x118, 0xf>(x);
+  x = dpp_max<0x142, 0xa>(x);   // row_bcast:15 into rows 1 and 3
+  x = dpp_max<0x143, 0xc>(x);   // row_bcast:31 into rows 2 and 3
+  const unsigned long long v = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_readlane((int)v, 63), hi = __builtin_amdgcn_readlane((int)(v >> 32), 63);
+  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+}
+__device__ __forceinline__ double read_lane(double x, int lane) {   // lane uniform
+  const unsigned long long v = __builtin_bit_cast(unsigned long long, x);
+  const unsigned lo = __builtin_amdgcn_readlane((int)v, lane), hi = __builtin_amdgcn_readlane((int)(v >> 32), lane);
+  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
 }
 
 // One panel of micro iterations (chol2_Lj + D update + BatchMax,
@@ -232,37 +227,75 @@ __device__ void wg_argmax_1024(double &k, double &v, int &i) {
 // by a workgroup of MICRO_ROWS lanes (lane i = batch row i):
 //   L(i, j) = (A(i, e) - sum_{p0 <= q < j} L(i, q) L(e, q)) / sqrt(D(e)),
 //   D(i) -= L(i, j)^2,  e <- first maximum of D (quantized keys).
-// (j, e, val) carry the loop state; lp[step][i] receives the panel's columns.
-__device__ void micro_panel_steps(double (&lp)[MICRO_PANEL][MICRO_ROWS], const double *__restrict__ A,
-                                  double *__restrict__ Lb, double *__restrict__ Db, long long nb, int nsteps,
-                                  double dmin, double inv_delta, int *__restrict__ piv, int &j, int &e, double &val,
-                                  int &done) {
-  const int i = threadIdx.x;
+// (j, e, val) carry the loop state; lp[step][i] receives the panel's columns,
+// d is row i's diagonal.
+//
+// A step is one chain: the column of A (written by other dies' CUs, so from the
+// last-level cache), the panel's terms, the diagonal, the maximum.  It is kept
+// short: the row's own terms stay in registers, the column's load is under way
+// while the root and the earlier terms are fetched, the maximum of the keys
+// goes through row operations and one LDS slot per wave (the wave's first row
+// that holds it by a ballot), and one barrier publishes slots and panel column
+// together (slots of alternate steps are separate).  42 us a panel of 1000
+// rows with shuffled (key, value, index) triples and five barriers a step.
+struct MicroSlots {
+  double key[2][MICRO_ROWS / 64], val[2][MICRO_ROWS / 64];
+  int row[2][MICRO_ROWS / 64];
+};
+__device__ void micro_panel_steps(double (&lp)[MICRO_PANEL][MICRO_ROWS], MicroSlots &S, const double *__restrict__ A,
+                                  double *__restrict__ Lb, double &d, long long nb, int nsteps, double dmin,
+                                  double inv_delta, int *__restrict__ piv, int &j, int &e, double &val, int &done) {
+  const int i = threadIdx.x, lane = i & 63, w = i >> 6;
   const bool row = i < nb;
+  const double *Ai = A + (row ? i : 0);
+  double l[MICRO_PANEL];
+  const int p0 = j;
   done = 0;
+#pragma unroll
   for (int step = 0; step < MICRO_PANEL; ++step) {
-    const double sq = sqrt(val);
-    double bk = inv_delta > 0.0 ? qabs(-1.0, inv_delta) : -1.0, bv = -1.0;
-    int bi = -1;
-    if (row) {
-      double s = A[i + nb * e];
-      for (int q = 0; q < step; ++q) s -= lp[q][i] * lp[q][e];
-      const double l = s / sq;
-      lp[step][i] = l;
-      Lb[i + nb * j] = l;
-      const double d = Db[i] - l * l;
-      Db[i] = d;
-      bk = inv_delta > 0.0 ? qabs(d, inv_delta) : d;
-      bv = d;
-      bi = i;
+    if (!done) {
+      e = __builtin_amdgcn_readfirstlane(e);
+      double s = Ai[nb * e];
+      // s / sqrt(val) as s y + (s - (s y) sqrt(val)) y with y = 1 / sqrt(val): the
+      // correctly rounded quotient (Markstein 1990), its reciprocal off the chain
+      const double sq = sqrt(val), y = 1.0 / sq;
+      double t[MICRO_PANEL];
+#pragma unroll
+      for (int q = 0; q < step; ++q) t[q] = lp[q][e];
+#pragma unroll
+      for (int q = 0; q < step; ++q) s -= l[q] * t[q];
+      const double l0 = s * y;
+      l[step] = fma(fma(-l0, sq, s), y, l0);
+      lp[step][i] = l[step];
+      d -= l[step] * l[step];
+      const double k = row ? (inv_delta > 0.0 ? qabs(d, inv_delta) : d) : -INFINITY;
+      const double kw = wave_max(k);
+      const unsigned long long has = __ballot(row && k == kw);
+      const int first = has ? (int)__ffsll(has) - 1 : 0;
+      if (lane == 0) {
+        S.key[step & 1][w] = has ? kw : -INFINITY;
+        S.row[step & 1][w] = has ? 64 * w + first : -1;
+      }
+      if (lane == first) S.val[step & 1][w] = d;
+      if (i == 0) piv[j] = e;
+      ++j;
+      __syncthreads();   // slots and panel column
+      // every wave picks the workgroup's first maximum: waves hold ascending rows
+      const int sl = lane & 15;
+      const double ks = S.key[step & 1][sl], vs = S.val[step & 1][sl];
+      const int rs = S.row[step & 1][sl];
+      const double km = wave_max(rs >= 0 ? ks : -INFINITY);
+      const unsigned long long hw = __ballot(rs >= 0 && ks == km) & 0xffffull;
+      const int ws = hw ? (int)__ffsll(hw) - 1 : 0;
+      e = hw ? __builtin_amdgcn_readlane(rs, ws) : -1;
+      val = read_lane(vs, ws);
+      done = (e < 0 || val <= dmin || j >= nb || j >= nsteps) ? 1 : 0;
     }
-    wg_argmax_1024(bk, bv, bi);   // its barriers also publish the panel column
-    if (threadIdx.x == 0) piv[j] = e;
-    ++j;
-    e = bi;
-    val = bv;
-    done = (bi < 0 || bv <= dmin || j >= nb || j >= nsteps) ? 1 : 0;
-    if (done) break;
+  }
+  if (row) {
+#pragma unroll
+    for (int step = 0; step < MICRO_PANEL; ++step)
+      if (p0 + step < j) Lb[i + nb * (p0 + step)] = l[step];
   }
 }
 
@@ -271,14 +304,16 @@ __global__ void __launch_bounds__(MICRO_ROWS) k_micro_panel(MicroState *st, cons
                                                             long long nb, int nsteps, double dmin, double inv_delta,
                                                             int *__restrict__ piv) {
   __shared__ double lp[MICRO_PANEL][MICRO_ROWS];
-  __shared__ int s_done;
-  if (threadIdx.x == 0) s_done = st->done;
-  __syncthreads();
-  if (s_done) return;
-  int j = st->j, e = st->e, done = 0;
+  __shared__ MicroSlots S;
+  if (__builtin_amdgcn_readfirstlane(st->done)) return;
+  int j = __builtin_amdgcn_readfirstlane(st->j), e = __builtin_amdgcn_readfirstlane(st->e), done = 0;
   double val = st->val;
   const int p0 = j;
-  micro_panel_steps(lp, A, Lb, Db, nb, nsteps, dmin, inv_delta, piv, j, e, val, done);
+  double d = threadIdx.x < nb ? Db[threadIdx.x] : 0.0;
+  // every wave has read the state before one of them writes it at the end
+  __syncthreads();
+  micro_panel_steps(lp, S, A, Lb, d, nb, nsteps, dmin, inv_delta, piv, j, e, val, done);
+  if (threadIdx.x < nb) Db[threadIdx.x] = d;
   if (threadIdx.x == 0) {
     st->p0 = p0;
     st->j = j;
@@ -328,20 +363,21 @@ __global__ void __launch_bounds__(MICRO_ROWS) k_micro_all(MicroState *st, double
                                                           long long nb, int nsteps, double dmin, double inv_delta,
                                                           int *__restrict__ piv) {
   __shared__ double lp[MICRO_PANEL][MICRO_ROWS];
-  __shared__ int s_done;
-  if (threadIdx.x == 0) s_done = st->done;
-  __syncthreads();
-  if (s_done) return;
-  int j = st->j, e = st->e, done = 0, p0 = j;
+  __shared__ MicroSlots S;
+  if (__builtin_amdgcn_readfirstlane(st->done)) return;
+  int j = __builtin_amdgcn_readfirstlane(st->j), e = __builtin_amdgcn_readfirstlane(st->e), done = 0, p0 = j;
   double val = st->val;
+  double d = threadIdx.x < nb ? Db[threadIdx.x] : 0.0;
+  __syncthreads();
   const int npanel = (nsteps + MICRO_PANEL - 1) / MICRO_PANEL;
   for (int pnl = 0; pnl < npanel; ++pnl) {
     p0 = j;
-    micro_panel_steps(lp, A, Lb, Db, nb, nsteps, dmin, inv_delta, piv, j, e, val, done);
+    micro_panel_steps(lp, S, A, Lb, d, nb, nsteps, dmin, inv_delta, piv, j, e, val, done);
     if (done) break;
     micro_update_lds(lp, A, nb, j - p0);
     __syncthreads();   // A updated, lp free for the next panel
   }
+  if (threadIdx.x < nb) Db[threadIdx.x] = d;
   if (threadIdx.x == 0) {
     st->p0 = p0;
     st->j = j;
@@ -353,16 +389,37 @@ __global__ void __launch_bounds__(MICRO_ROWS) k_micro_all(MicroState *st, double
 
 // A(i, c) -= sum_{q = p0}^{j-1} L(i, q) L(c, q) for the panel just finished
 // (skipped once the loop has stopped: A is not read again).
-__global__ void k_micro_update(const MicroState *st, double *__restrict__ A, const double *__restrict__ Lb,
-                               long long nb) {
+// 64 x 64 elements per workgroup, the panel's rows in LDS, sixteen columns a
+// lane: A is read and written once (the element-per-lane form fetched 32 panel
+// values for each: 11 us at 1000 rows).
+__global__ void __launch_bounds__(256) k_micro_update(const MicroState *st, double *__restrict__ A,
+                                                      const double *__restrict__ Lb, long long nb) {
   if (st->done) return;
-  const int p0 = st->p0, j = st->j;
-  const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  const long long c = blockIdx.y;
-  if (i >= nb || c >= nb) return;
-  double s = A[i + nb * c];
-  for (int q = p0; q < j; ++q) s -= Lb[i + nb * q] * Lb[c + nb * q];
-  A[i + nb * c] = s;
+  __shared__ double s_r[MICRO_PANEL][64], s_c[MICRO_PANEL][64];
+  const int p0 = st->p0, np = st->j - p0;
+  const long long i0 = blockIdx.x * 64LL, c0 = blockIdx.y * 64LL;
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+  double a[16];   // row i0 + x, columns c0 + 16 y ..
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    const long long cc = c0 + 16 * y + c;
+    a[c] = (i0 + x < nb && cc < nb) ? A[i0 + x + nb * cc] : 0.0;
+  }
+  for (int q = y; q < np; q += 4) {
+    s_r[q][x] = i0 + x < nb ? Lb[i0 + x + nb * (p0 + q)] : 0.0;
+    s_c[q][x] = c0 + x < nb ? Lb[c0 + x + nb * (p0 + q)] : 0.0;
+  }
+  __syncthreads();
+  for (int q = 0; q < np; ++q) {
+    const double r = s_r[q][x];
+#pragma unroll
+    for (int c = 0; c < 16; ++c) a[c] -= r * s_c[q][16 * y + c];
+  }
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    const long long cc = c0 + 16 * y + c;
+    if (i0 + x < nb && cc < nb) A[i0 + x + nb * cc] = a[c];
+  }
 }
 
 // D(bd(piv(q))) = 0 for the pivots of this macro iteration (precision form)
@@ -388,26 +445,38 @@ __global__ void k_build_lp(double *__restrict__ LP, long long J, const double *_
   if (q < J && r < J) LP[q + J * r] = (r <= q) ? Lb[piv[q] + nb * r] : 0.0;
 }
 
-// batch rows keep the values of the sequential recurrence; then
-// D(i) -= L(i, j0+q)^2 for q = 0..J-1 in order
-__global__ void k_finish_rows(double *__restrict__ Lt, long long ldL, long long j0, long long J,
-                              const double *__restrict__ Lb, long long nb, const long long *__restrict__ bd,
-                              double *__restrict__ D, long long nrows) {
-  long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (e < nb)
-    for (long long q = 0; q < J; ++q) Lt[bd[e] + ldL * (j0 + q)] = Lb[e + nb * q];
+// batch rows keep the values of the sequential recurrence
+__global__ void k_finish_rows(double *__restrict__ Lt, long long ldL, long long j0, const double *__restrict__ Lb,
+                              long long nb, const long long *__restrict__ bd) {
+  const long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x, q = blockIdx.y;
+  if (e < nb) Lt[bd[e] + ldL * (j0 + q)] = Lb[e + nb * q];
 }
 
-__global__ void k_update_d(const double *__restrict__ Lt, long long ldL, long long j0, long long J,
-                           double *__restrict__ D, long long nrows) {
-  long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-  if (i >= nrows) return;
-  double d = D[i];
-  for (long long q = 0; q < J; ++q) {
-    const double l = Lt[i + ldL * (j0 + q)];
-    d = d - l * l;
+// D(i) -= L(i, j0+q)^2 for q = 0..J-1 in order.  64 rows per workgroup; four
+// waves bring 64 columns at a time into LDS, so that the loads overlap while
+// the subtractions keep their order (a lane walking its row's columns waited
+// for its own loads: 40 us at 300 columns).
+__global__ void __launch_bounds__(256) k_update_d(const double *__restrict__ Lt, long long ldL, long long j0,
+                                                  long long J, double *__restrict__ D, long long nrows) {
+  __shared__ double s_l[64][64];
+  const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
+  const long long i = blockIdx.x * 64LL + x;
+  const bool ok = i < nrows;
+  double d = ok && y == 0 ? D[i] : 0.0;
+  for (long long q0 = 0; q0 < J; q0 += 64) {
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      const long long q = q0 + 16 * y + k;
+      s_l[16 * y + k][x] = ok && q < J ? Lt[i + ldL * (j0 + q)] : 0.0;   // zeros change nothing
+    }
+    __syncthreads();
+    if (y == 0) {
+#pragma unroll 16
+      for (int q = 0; q < 64; ++q) d = d - s_l[q][x] * s_l[q][x];
+    }
+    __syncthreads();
   }
-  D[i] = d;
+  if (ok && y == 0) D[i] = d;
 }
 
 __global__ void k_blockmax(const double *__restrict__ D, long long n, double *__restrict__ part) {
@@ -448,130 +517,173 @@ __global__ void k_zero_pad_rows(double *__restrict__ W, long long ldw, long long
     for (long long r = r0 + threadIdx.x; r < r1; r += blockDim.x) W[r + ldw * c] = 0.0;
 }
 
+// One level of the inverse's merge in LDS, H = 8, 16, 32: for every pair of
+// H x H diagonal blocks [A 0; B C]^-1 = [A^-1 0; -C^-1 (B A^-1) C^-1].  A lane
+// forms 2 x 2 elements (one at H = 8, where there are as many elements as
+// lanes); the sums run over the whole block, so that every load is known in
+// advance (the zeros above a diagonal change nothing).
+template <int H>
+__device__ __forceinline__ void leaf_merge(const double (*s)[POTF_NB + 1], double (*x)[POTF_NB + 1], double *t,
+                                           int tid) {
+  constexpr int T = H == 8 ? 1 : 2, HT = H / T;
+  constexpr int NPR = POTF_NB / (2 * H), NE = NPR * HT * HT;   // 256, 128 or 256 lanes
+  const int pr = tid / (HT * HT), ij = tid % (HT * HT), i = ij % HT * T, j = ij / HT * T;
+  const int a0 = 2 * H * pr, c0 = a0 + H;
+  if (tid < NE) {
+    double acc[T][T];
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+#pragma unroll
+      for (int v = 0; v < T; ++v) acc[u][v] = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < H; ++k)
+#pragma unroll
+      for (int u = 0; u < T; ++u)
+#pragma unroll
+        for (int v = 0; v < T; ++v) acc[u][v] += s[c0 + i + u][a0 + k] * x[a0 + k][a0 + j + v];
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+#pragma unroll
+      for (int v = 0; v < T; ++v) t[pr * H * H + (i + u) + H * (j + v)] = acc[u][v];
+  }
+  __syncthreads();
+  if (tid < NE) {
+    double acc[T][T];
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+#pragma unroll
+      for (int v = 0; v < T; ++v) acc[u][v] = 0.0;
+#pragma unroll 8
+    for (int k = 0; k < H; ++k)
+#pragma unroll
+      for (int u = 0; u < T; ++u)
+#pragma unroll
+        for (int v = 0; v < T; ++v) acc[u][v] += x[c0 + i + u][c0 + k] * t[pr * H * H + k + H * (j + v)];
+#pragma unroll
+    for (int u = 0; u < T; ++u)
+#pragma unroll
+      for (int v = 0; v < T; ++v) x[c0 + i + u][a0 + j + v] = -acc[u][v];
+  }
+  __syncthreads();
+}
+
 // Cholesky factor L and its inverse X of the diagonal block at k0 (b <= POTF_NB
 // rows, lower triangle of V read); writes L (zero above the diagonal) over the
 // block of V and X into the block of X.  Does nothing once an earlier block failed.
+//
+// The leaves follow each other (every split waits for its first half), so a
+// leaf is latency: 64 columns, each a root, a quotient and an exchange.  Lane r
+// of every wave holds row r, the columns are dealt out to the four waves, and
+// one barrier publishes a scaled column.  The wave that owns the next column
+// updates that one alone before its root, and makes up for the others after
+// the barrier, while the next owner is at its own: per column only a
+// broadcast, one update, root, quotient and store are in line.  66 us a leaf of
+// 64 rows with 4 x 4 tiles, two barriers a column and merges with run-time
+// bounds, 37 us here; the operations on each element and their order are the
+// same.
 __global__ void __launch_bounds__(256) k_chol_inv_leaf(double *__restrict__ V, double *__restrict__ X, long long n,
                                                        long long k0, int b, int *__restrict__ info) {
   __shared__ double s[POTF_NB][POTF_NB + 1];
   __shared__ double x[POTF_NB][POTF_NB + 1];
-  __shared__ double t[POTF_NB * POTF_NB / 2];   // B A^-1 of the merge step
-  __shared__ int s_info;
-  const int tid = threadIdx.x;
-  if (tid == 0) s_info = *info;
-  __syncthreads();
-  if (s_info != 0) return;
-  // factorization in registers: thread (tr, tc) of a 16 x 16 grid holds the
-  // 4 x 4 tile of rows 4 tr .. 4 tr + 3 and columns 4 tc .. 4 tc + 3 (tiles
-  // above the diagonal idle); per column j the diagonal goes through LDS, the
-  // owners of column j scale it and publish it, every tile takes its rank-1
-  // update: two barriers per column.  The block is padded with an identity.
-  const int tr = tid & 15, tc = tid >> 4;
-  double a[4][4];
+  __shared__ double t[POTF_NB * POTF_NB / 2];   // B A^-1 of the merge steps
+  __shared__ double cl[POTF_NB + 1][POTF_NB];   // scaled columns (the last row is only read for columns past the end)
+  __shared__ int s_bad;
+  const int tid = threadIdx.x, r = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a[m]: row r of column 4 (m + jb) + w; the block is padded with an identity.
+  // The registers move down after every four columns, so that the loop stays
+  // rolled: unrolled it is 70 KB of code run once per leaf.
+  constexpr int NM = POTF_NB / 4;
+  double a[NM];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int r = 4 * tr + i, c = 4 * tc + jj;
-      a[i][jj] = (r < b && c < b && r >= c) ? V[(k0 + r) + n * (k0 + c)] : (r == c ? 1.0 : 0.0);
-    }
-  for (int e = tid; e < POTF_NB * POTF_NB; e += 256) x[e % POTF_NB][e / POTF_NB] = 0.0;
-  __shared__ double s_d;
-  __shared__ double s_col[POTF_NB];
-  int jend = b;
-  for (int j = 0; j < b; ++j) {
-    const int tj = j >> 2;
-    if (tr == tj && tc == tj) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if ((j & 3) == i) s_d = a[i][i];
-    }
-    __syncthreads();
-    const double d = s_d;
-    if (!(d > 0.0)) {   // the same LDS value in every lane: a uniform exit
-      jend = j;
-      break;
-    }
-    const double sq = sqrt(d);
-    if (tc == tj && tr >= tj) {
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
-        if ((j & 3) == jj) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int r = 4 * tr + i;
-            if (r == j) a[i][jj] = sq;
-            else if (r > j) a[i][jj] = a[i][jj] / sq;
-            if (r >= j) s_col[r] = a[i][jj];
-          }
-        }
-    }
-    __syncthreads();
-    if (tr >= tc && 4 * tr + 3 > j) {
-      double cr[4], cc[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        cr[i] = s_col[4 * tr + i];
-        cc[i] = s_col[4 * tc + i];
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) {
-          const int r = 4 * tr + i, c = 4 * tc + jj;
-          if (c > j && r >= c) a[i][jj] -= cr[i] * cc[jj];
-        }
-    }
+  for (int m = 0; m < NM; ++m) {
+    const int c = 4 * m + w;
+    a[m] = (r < b && c < b && r >= c) ? V[(k0 + r) + n * (k0 + c)] : (r == c ? 1.0 : 0.0);
   }
-  if (jend < b) {
-    if (tid == 0) *info = (int)(k0 + jend + 1);
+  const int failed = *info;   // set by an earlier leaf, so the same in every lane
+  for (int e = tid; e < POTF_NB * POTF_NB; e += 256) x[e % POTF_NB][e / POTF_NB] = 0.0;
+  if (tid == 0) s_bad = POTF_NB;
+  __syncthreads();
+  if (failed != 0) return;
+  // column j from the owner's value v of it
+  auto scale = [&](double v, int j) {
+    const double d = read_lane(v, j);
+    const double sq = sqrt(d);
+    v = v / sq;
+    if (r == j) v = sq;
+    if (r < j) v = 0.0;
+    cl[j][r] = v;
+    if (r == 0 && !(d > 0.0) && s_bad == POTF_NB) s_bad = j;
+    return v;
+  };
+  if (w == 0) a[0] = scale(a[0], 0);
+  __syncthreads();
+#pragma unroll 1
+  for (int jb = 0; jb < NM; ++jb) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = 4 * jb + u;
+      const double *col = cl[j];
+      const double cr = col[r];
+      const bool own = w == ((u + 1) & 3);   // of column j + 1: a[0], or a[1] of wave 0 at the end of the group
+      // rows above a column's diagonal take the update too: they are not read
+      auto rest = [&]() {
+        // a[m] of a column past the end takes whatever stands there and is not read
+        const double *cw = col + 4 * jb + w;
+        double cc[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) cc[m] = cw[4 * m];
+        if (w > u && !own) a[0] -= cr * cc[0];
+        if (u < 3 || !own) a[1] -= cr * cc[1];
+#pragma unroll
+        for (int m = 2; m < NM; ++m) a[m] -= cr * cc[m];
+      };
+      if (own && j + 1 < POTF_NB) {
+        if (u < 3) {
+          a[0] -= cr * col[j + 1];
+          a[0] = scale(a[0], j + 1);
+        } else {
+          a[1] -= cr * col[j + 1];
+          a[1] = scale(a[1], j + 1);
+        }
+      }
+      if (!own) rest();
+      __syncthreads();
+      if (own) rest();
+    }
+    s[r][4 * jb + w] = a[0];
+#pragma unroll
+    for (int m = 0; m + 1 < NM; ++m) a[m] = a[m + 1];
+    a[NM - 1] = 0.0;
+  }
+  const int jbad = s_bad;
+  if (jbad < b) {
+    if (tid == 0) *info = (int)(k0 + jbad + 1);
     return;
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) s[4 * tr + i][4 * tc + jj] = a[i][jj];
   __syncthreads();
-  // X = L^-1 (L padded to POTF_NB rows with an identity): the eight 8 x 8
-  // diagonal blocks by forward substitution, one column per lane, then pairs
-  // of blocks merged, [A 0; B C]^-1 = [A^-1 0; -C^-1 (B A^-1) C^-1], for
-  // h = 8, 16, 32, each product spread over all lanes (short dependency chains)
+  // X = L^-1: the eight 8 x 8 diagonal blocks by forward substitution, one
+  // column per lane, then pairs of blocks merged
   if (tid < POTF_NB) {
     const int r0 = (tid / 8) * 8, c = tid % 8;
-    x[r0 + c][r0 + c] = 1.0 / s[r0 + c][r0 + c];
-    for (int r = c + 1; r < 8; ++r) {
+    double xs[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
       double acc = 0.0;
-      for (int k = c; k < r; ++k) acc += s[r0 + r][r0 + k] * x[r0 + k][r0 + c];
-      x[r0 + r][r0 + c] = -acc / s[r0 + r][r0 + r];
+#pragma unroll
+      for (int k = 0; k < i; ++k) acc += s[r0 + i][r0 + k] * xs[k];   // xs[k] = 0 for k < c
+      xs[i] = i < c ? 0.0 : (i == c ? 1.0 : -acc) / s[r0 + i][r0 + i];
+      x[r0 + i][r0 + c] = xs[i];
     }
   }
   __syncthreads();
-  for (int h = 8; h < POTF_NB; h *= 2) {
-    const int npair = POTF_NB / (2 * h);
-    // T = B A^-1 for every pair (A^-1 lower triangular)
-    for (int e = tid; e < npair * h * h; e += 256) {
-      const int pr = e / (h * h), ij = e % (h * h), i = ij % h, j = ij / h;
-      const int a0 = 2 * h * pr, c0 = a0 + h;
-      double acc = 0.0;
-      for (int k = j; k < h; ++k) acc += s[c0 + i][a0 + k] * x[a0 + k][a0 + j];
-      t[e] = acc;
+  leaf_merge<8>(s, x, t, tid);
+  leaf_merge<16>(s, x, t, tid);
+  leaf_merge<32>(s, x, t, tid);
+  for (int c = w; c < b; c += 4)
+    if (r < b) {
+      V[(k0 + r) + n * (k0 + c)] = r >= c ? s[r][c] : 0.0;
+      X[(k0 + r) + n * (k0 + c)] = r >= c ? x[r][c] : 0.0;
     }
-    __syncthreads();
-    // X21 = -C^-1 T (C^-1 lower triangular)
-    for (int e = tid; e < npair * h * h; e += 256) {
-      const int pr = e / (h * h), ij = e % (h * h), i = ij % h, j = ij / h;
-      const int a0 = 2 * h * pr, c0 = a0 + h;
-      double acc = 0.0;
-      for (int k = 0; k <= i; ++k) acc += x[c0 + i][c0 + k] * t[pr * h * h + k + h * j];
-      x[c0 + i][a0 + j] = -acc;
-    }
-    __syncthreads();
-  }
-  for (int e = tid; e < b * b; e += 256) {
-    const int r = e % b, c = e / b;
-    V[(k0 + r) + n * (k0 + c)] = r >= c ? s[r][c] : 0.0;
-    X[(k0 + r) + n * (k0 + c)] = r >= c ? x[r][c] : 0.0;
-  }
 }
 
 // ------------------------------------------------------------------ helpers
@@ -1126,8 +1238,8 @@ void chol_build(Context &C, double tau, double kappa, long long max_block_dim, l
           for (int k = 0; k < 4 && pnl < npanel_max; ++k, ++pnl) {
             hipLaunchKernelGGL(k_micro_panel, dim3(1), dim3(MICRO_ROWS), 0, C.stream, dstate.p, dMb.p, dLb.p,
                                dDb.p, nb, nsteps, dmin, qd, dpiv.p);
-            hipLaunchKernelGGL(k_micro_update, dim3((unsigned)((nb + 255) / 256), (unsigned)nb), dim3(256), 0,
-                               C.stream, dstate.p, dMb.p, dLb.p, nb);
+            hipLaunchKernelGGL(k_micro_update, dim3((unsigned)((nb + 63) / 64), (unsigned)((nb + 63) / 64)), dim3(256),
+                               0, C.stream, dstate.p, dMb.p, dLb.p, nb);
           }
           MicroState hs{};
           C.read(&hs, dstate.p, sizeof(hs));
@@ -1153,10 +1265,10 @@ void chol_build(Context &C, double tau, double kappa, long long max_block_dim, l
           ROCBLAS_CHECK(rocblas_dtrsm(C.blas, rocblas_side_right, rocblas_fill_lower, rocblas_operation_transpose,
                                       rocblas_diagonal_non_unit, ncand, J, &one, dLP.p, J,
                                       dL.p + (size_t)ncand * j0, ncand));
-          hipLaunchKernelGGL(k_finish_rows, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, C.stream, dL.p, ncand,
-                             j0, J, dLb.p, nb, dbd.p, dD.p, ncand);
-          hipLaunchKernelGGL(k_update_d, dim3((unsigned)((ncand + 255) / 256)), dim3(256), 0, C.stream, dL.p,
-                             ncand, j0, J, dD.p, ncand);
+          hipLaunchKernelGGL(k_finish_rows, dim3((unsigned)((nb + 255) / 256), (unsigned)J), dim3(256), 0, C.stream,
+                             dL.p, ncand, j0, dLb.p, nb, dbd.p);
+          hipLaunchKernelGGL(k_update_d, dim3((unsigned)((ncand + 63) / 64)), dim3(256), 0, C.stream, dL.p, ncand, j0,
+                             J, dD.p, ncand);
           if (split)
             hipLaunchKernelGGL(k_zero_pivot_d, dim3((unsigned)((J + 255) / 256)), dim3(256), 0, C.stream, dD.p,
                                dbd.p, dpiv.p, J);

@@ -21,6 +21,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstdio>
+#include "crt.h"
 #include "gi_context.h"
 
 namespace gi {
@@ -1190,7 +1191,9 @@ void chol_build(Context &C, double tau, double kappa, long long max_block_dim, l
         if (flags & 16)
           split_bf16_gemm(C, rocblas_operation_none, rocblas_operation_transpose, ncand, nops_batch, nchol, alpha,
                           dL.p, ncand, dLB.p, nops_batch, beta, dM.p, ncand);
-        else
+        else if (!crt_pays(ncand, nops_batch, nchol) ||
+                 !crt_gemm_nt(C, ncand, nops_batch, nchol, alpha, dL.p, ncand, dLB.p, nops_batch, beta, dM.p, ncand,
+                              false))
           ROCBLAS_CHECK(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, ncand,
                                       nops_batch, nchol, &alpha, dL.p, ncand, dLB.p, nops_batch, &beta, dM.p, ncand));
         C.wait();
@@ -1463,15 +1466,19 @@ void chol_build(Context &C, double tau, double kappa, long long max_block_dim, l
       const double one = 1.0, zero = 0.0;
       // Block rows hold a multiple of 128 rows (the DGEMM macro tile), counted
       // from the last row: only the first block, whose product is the
-      // shortest (k = r1), has a partly filled tile row.
-      const long long nblk = std::max<long long>(1, std::min<long long>(C.vec_blocks, nvec / 256));
-      const long long rows_blk = std::max<long long>(128, (nvec + 64 * nblk) / (128 * nblk) * 128);
-      for (long long r1 = nvec; r1 > 0;) {
-        const long long r0 = std::max<long long>(0, r1 - rows_blk);
-        ROCBLAS_CHECK(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, r1 - r0, ldw, r1,
-                                    &one, S.inv_l.p + r0, nvec, dW.p, ldw, &zero,
-                                    S.rkpq.p + (size_t)(X0 - 1) * nvec * msd + r0, nvec));
-        r1 = r0;
+      // shortest (k = r1), has a partly filled tile row.  Large products go to
+      // the int8 matrix cores instead (crt.hip), triangular by its tiles.
+      double *const dst = S.rkpq.p + (size_t)(X0 - 1) * nvec * msd;
+      if (!crt_pays(nvec, ldw, nvec, 0.5 + 128.0 / (double)nvec) ||
+          !crt_gemm_nt(C, nvec, ldw, nvec, one, S.inv_l.p, nvec, dW.p, ldw, zero, dst, nvec, true)) {
+        const long long nblk = std::max<long long>(1, std::min<long long>(C.vec_blocks, nvec / 256));
+        const long long rows_blk = std::max<long long>(128, (nvec + 64 * nblk) / (128 * nblk) * 128);
+        for (long long r1 = nvec; r1 > 0;) {
+          const long long r0 = std::max<long long>(0, r1 - rows_blk);
+          ROCBLAS_CHECK(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, r1 - r0, ldw, r1,
+                                      &one, S.inv_l.p + r0, nvec, dW.p, ldw, &zero, dst + r0, nvec));
+          r1 = r0;
+        }
       }
       C.wait();
       t_gemm += now() - tg;

@@ -51,6 +51,7 @@ Context::~Context() {
   release_chol_work(*this);
   release_thc_work(*this);
   release_grad_work(*this);
+  release_crt_work(*this);
   for (int i = 0; i < 2; ++i) {
     spl_slices[i].release();
     spl_exp[i].release();

@@ -89,6 +89,7 @@ struct CholState {
 
 struct CholWork;   // gi_chol_build work arrays (chol.hip)
 struct ThcWork;    // work arrays of the THC calls (thc.hip)
+struct CrtWork;    // work arrays of the int8 products (crt.hip)
 struct GradWork;   // work arrays of the Coulomb energy and gradient (grad.hip)
 
 struct Context {
@@ -139,6 +140,8 @@ struct Context {
   ThcWork *thcw = nullptr;
   // device work arrays of the Coulomb energy and gradient (grad.hip), grow-only
   GradWork *gradw = nullptr;
+  // device work arrays of the int8 products (crt.hip), grow-only
+  CrtWork *crtw = nullptr;
   // split-BF16 products (split.hip): BF16 slice planes and per-chunk row
   // scale exponents of the two operands; grow-only, kept across calls
   DBuf<unsigned short> spl_slices[2];
@@ -295,6 +298,7 @@ void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_t
                      long long block_dim, std::vector<long long> &pivots, long long &nred);
 void release_thc_work(Context &C);
 void release_grad_work(Context &C);
+void release_crt_work(Context &C);
 
 // Coulomb energy of a density and its nuclear gradient (grad.hip)
 void coulomb_energy_grad(Context &C, const double *D, long long ldd, double kappa, double *energy,

@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <cmath>
 #include <rocsolver/rocsolver.h>
+#include "crt.h"
 #include "gi_context.h"
 
 namespace gi {
@@ -374,14 +375,18 @@ void thc_z(Context &C, const double *dX, long long ldx, long long npts, long lon
   std::vector<int> colpq;
   thc_column_pairs(C, colpq);
   w.colpq.upload(colpq, C.stream);
-  // XR = 2 Xgpq R^T in column chunks of at most 2^26 doubles of Xgpq
+  // XR = 2 Xgpq R^T: on the int8 matrix cores where that pays (crt.hip; the
+  // products X(g,p) X(g,q) then never reach memory), else as DGEMMs over column
+  // chunks of at most 2^26 doubles of Xgpq
   const long long nc = std::max<long long>(1, std::min<long long>(ncols, (1LL << 26) / npts));
-  w.W.alloc((size_t)(npts * nc));
   const double two = 2.0, one = 1.0, zero = 0.0;
+  const bool crt = crt_pays(npts, nvec, ncols) &&
+                   crt_pairs_nt(C, npts, nvec, ncols, two, dX, ldx, w.colpq.p, S.rkpq.p, nvec, zero, dZ, ldz);
+  if (!crt) w.W.alloc((size_t)(npts * nc));
   const dim3 gp((unsigned)((npts + 255) / 256), ygrid(nc));
   if (ncols == 0 || nvec == 0)
     GI_HIP(hipMemset2DAsync(dZ, sizeof(double) * ldz, 0, sizeof(double) * npts, nvec, C.stream));
-  for (long long c0 = 0; c0 < ncols && nvec > 0; c0 += nc) {
+  for (long long c0 = 0; !crt && c0 < ncols && nvec > 0; c0 += nc) {
     const long long m = std::min(nc, ncols - c0);
     hipLaunchKernelGGL(k_thc_xgpq, gp, dim3(256), 0, C.stream, dX, ldx, npts, w.colpq.p, c0, m, w.W.p);
     GI_HIP(hipGetLastError());

@@ -30,6 +30,7 @@
 #include <rocsolver/rocsolver.h>
 #include "crt.h"
 #include "gi_context.h"
+#include "gi_wave.h"
 
 namespace gi {
 
@@ -52,7 +53,7 @@ struct ThcWork {
   // gathers into the other), step state, pivots in order
   DBuf<double> pxyz, pX, pD, pD2, pL[2], pS[2];
   DBuf<long long> pcand, pmap, ppiv;
-  DBuf<unsigned char> pstate;
+  DBuf<unsigned char> pstate, pmax;
 };
 static ThcWork &thc_work(Context &C) {
   if (!C.thcw) C.thcw = new ThcWork();
@@ -160,86 +161,117 @@ struct PivotState {
   int pad;
 };
 
-// One pivot step, launched with vector index k.  Every workgroup finds the
-// step's pivot itself, the first candidate index of the largest D (maxloc), so
-// that no workgroup waits for another; it is taken when D > thresh
-// (thc_Chol_NextBlock, TensorHypercontraction.f90:1012-1027), and workgroup 0
-// records it.  Then the vector over every candidate g (column k - lbase of L)
-//   on the fly (Sh == null): ((sum_p X(g,p) X(h,p))^2 - sum_j L(g,j) L(h,j)) / sqrt(D(h))
-//   Schur:                    (Sh(g,h) - sum_j L(g,j) L(h,j)) / sqrt(D(h))
-// and Dout(g) = Din(g) - L(g,k)^2: D is read from one buffer and written to the
-// other, so that the workgroups still searching see the step's input.  64
-// candidates per workgroup; the sixteen wavefronts split the sums.  A step
-// without a pivot sets done, and every later step of the block exits at once.
+// The largest D of 64 consecutive candidates and the first candidate that holds
+// it (-1: none), as every workgroup of a step leaves them for the next step.
+struct PivotMax {
+  double d;
+  long long g;
+};
+__device__ __forceinline__ PivotMax pivot_max(double d, bool ok, long long g0) {
+  const double m = wave_max(ok ? d : -INFINITY);
+  const unsigned long long has = __ballot(ok && d == m);
+  return PivotMax{m, has ? g0 + __ffsll(has) - 1 : -1};
+}
+
+// maxima of D before the first step of a block
+__global__ void __launch_bounds__(64) k_thc_pivot_max(const double *__restrict__ D, long long ncand,
+                                                      PivotMax *__restrict__ E) {
+  const long long g0 = blockIdx.x * 64LL, g = g0 + threadIdx.x;
+  const PivotMax m = pivot_max(g < ncand ? D[g] : 0.0, g < ncand, g0);
+  if (threadIdx.x == 0) E[blockIdx.x] = m;
+}
+
+// One pivot step, launched with vector index k.  Every wave finds the step's
+// pivot itself, the first candidate index of the largest D (maxloc), from the
+// maxima that the workgroups of the step before have left (Ein), so that no
+// workgroup waits for another; it is taken when D > thresh (thc_Chol_NextBlock,
+// TensorHypercontraction.f90:1012-1027), and workgroup 0 records it.  Then the
+// vector over every candidate g (column k - lbase of L)
+//   on the fly: ((sum_p X(g,p) X(h,p))^2 - sum_j L(g,j) L(h,j)) / sqrt(D(h))
+//   Schur:      (Sh(g,h) - sum_j L(g,j) L(h,j)) / sqrt(D(h))
+// D(g) -= L(g,k)^2, and the workgroup's new maximum (Eout).  64 candidates per
+// workgroup; the sixteen wavefronts split the sums.  A step without a pivot sets
+// done, and every later step of the block exits at once.
+//
+// A step is a launch and two trips to memory: the maxima, the candidates' own
+// vector elements (which do not depend on the pivot, in the Schur form at most
+// PIV_PANEL / 16 a lane) and D travel together, then the pivot's row and column.
+// With the whole of D scanned by every workgroup, a tree of ten barriers and
+// the elements fetched after it a step took 11.8 us at 9600 candidates; 4.7 us
+// here, and about 2.5 us between two launches.  Pruning 9600 points (6000
+// pivots, 600 AOs): 92 -> 57 ms.
+constexpr int PIV_PANEL = 128;   // Schur form: vectors kept outside Shat
+template <bool SCHUR>
 __global__ void __launch_bounds__(1024) k_thc_pivot_step(const double *__restrict__ X, long long ncand,
                                                          long long nao, const double *__restrict__ Sh,
                                                          double *__restrict__ L, long long lbase, long long k,
-                                                         const double *__restrict__ Din, double *__restrict__ Dout,
+                                                         double *__restrict__ D, const PivotMax *__restrict__ Ein,
+                                                         PivotMax *__restrict__ Eout,
                                                          const long long *__restrict__ cand,
                                                          long long *__restrict__ piv, PivotState *st, double thresh,
                                                          double thresh_red) {
-  __shared__ double s_v[1024];
-  __shared__ long long s_i[1024];
+  constexpr int NJ = PIV_PANEL / 16;
   __shared__ double s1[16][64], s2[16][64];
-  const int t = threadIdx.x;
-  if (st->done) return;   // uniform: set by an earlier launch
-  double bv = -1.0;
-  long long bi = -1;
-  for (long long g = t; g < ncand; g += 1024) {
-    const double v = Din[g];
-    if (bi < 0 || v > bv) {   // strictly larger: the first index wins within a thread
-      bv = v;
-      bi = g;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const long long g = blockIdx.x * 64LL + lane, kl = k - lbase;
+  const bool ok = g < ncand;
+  const int done = st->done;   // set by an earlier launch
+  double lg[NJ];
+  if constexpr (SCHUR) {
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) lg[i] = ok && w + 16 * i < kl ? L[g + ncand * (w + 16 * i)] : 0.0;
+  }
+  const double d = ok && w == 0 ? D[g] : 0.0;
+  double bv = -INFINITY, bi = INFINITY;   // largest entry and its candidate (exact as a double)
+  for (int e = lane; e < (int)gridDim.x; e += 64) {
+    const PivotMax m = Ein[e];
+    if (m.g >= 0 && (m.d > bv || bi == INFINITY)) {   // entries of a lane ascend: the first index wins
+      bv = m.d;
+      bi = (double)m.g;
     }
   }
-  s_v[t] = bv;
-  s_i[t] = bi;
-  __syncthreads();
-  for (int off = 512; off > 0; off >>= 1) {
-    if (t < off) {
-      const double v2 = s_v[t + off];
-      const long long i2 = s_i[t + off];
-      if (i2 >= 0 && (s_i[t] < 0 || v2 > s_v[t] || (v2 == s_v[t] && i2 < s_i[t]))) {
-        s_v[t] = v2;
-        s_i[t] = i2;
-      }
-    }
-    __syncthreads();
-  }
-  const double dh = s_v[0];
-  const long long h = s_i[0];
-  if (!(h >= 0 && dh > thresh)) {   // uniform: the same LDS values in every lane
+  if (done) return;   // uniform
+  const double dh = wave_max(bv);
+  const double hd = -wave_max(bv == dh ? -bi : -INFINITY);
+  if (!(hd < INFINITY && dh > thresh)) {   // uniform: every wave of every workgroup reads the same entries
     if (blockIdx.x == 0 && t == 0) st->done = 1;
     return;
   }
+  const long long h = (long long)hd;
   if (blockIdx.x == 0 && t == 0) {
     piv[k] = cand[h];
     st->npiv = k + 1;
     if (dh > thresh_red) st->nred = k + 1;
   }
-  const long long kl = k - lbase;
-  const int lane = t & 63, w = t >> 6;
-  const long long g = blockIdx.x * 64LL + lane;
-  double a = 0.0, c = 0.0;
-  if (g < ncand) {
-    if (!Sh)
-      for (long long p = w; p < nao; p += 16) a += X[g + ncand * p] * X[h + ncand * p];
+  double a = 0.0, c = 0.0, col = 0.0;
+  if constexpr (SCHUR) {
+    const int j = w + 16 * (lane & (NJ - 1));
+    const double lh = j < kl ? L[h + ncand * j] : 0.0;   // lane i: the pivot's element of this wave's term i
+    if (w == 0 && ok) col = Sh[g + ncand * h];
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) c += lg[i] * read_lane(lh, i);
+  } else if (ok) {
+    for (long long p = w; p < nao; p += 16) a += X[g + ncand * p] * X[h + ncand * p];
     for (long long j = w; j < kl; j += 16) c += L[g + ncand * j] * L[h + ncand * j];
+    s1[w][lane] = a;
   }
-  s1[w][lane] = a;
   s2[w][lane] = c;
   __syncthreads();
-  if (w == 0 && g < ncand) {
-    double sg = 0.0, lg = 0.0;
+  if (w == 0) {
+    double sg = 0.0, ls = 0.0;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      sg += s1[i][lane];
-      lg += s2[i][lane];
+      if constexpr (!SCHUR) sg += s1[i][lane];
+      ls += s2[i][lane];
     }
-    const double col = Sh ? Sh[g + ncand * h] : sg * sg;
-    const double v = (col - lg) / sqrt(dh);
-    L[g + ncand * kl] = v;
-    Dout[g] = Din[g] - v * v;
+    if constexpr (!SCHUR) col = sg * sg;
+    const double v = (col - ls) / sqrt(dh), dn = d - v * v;
+    if (ok) {
+      L[g + ncand * kl] = v;
+      D[g] = dn;
+    }
+    const PivotMax m = pivot_max(dn, ok, blockIdx.x * 64LL);
+    if (lane == 0) Eout[blockIdx.x] = m;
   }
 }
 
@@ -505,6 +537,8 @@ void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_t
   w.pD2.alloc((size_t)npts);
   double *const Dbuf[2] = {w.pD.p, w.pD2.p};
   int dcur = 0;   // the buffer holding the current residual diagonal
+  w.pmax.alloc(sizeof(PivotMax) * 2 * (size_t)((npts + 63) / 64));
+  PivotMax *const Ebuf[2] = {(PivotMax *)w.pmax.p, (PivotMax *)w.pmax.p + (npts + 63) / 64};
   w.ppiv.alloc((size_t)npts);
   w.pstate.alloc(sizeof(PivotState));
   w.pxyz.alloc((size_t)(3 * npts));
@@ -515,7 +549,6 @@ void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_t
   PivotState *dst = (PivotState *)w.pstate.p;
   int cur = 0, scur = 0;
   bool converged = false, schur = false;
-  long long lbase = 0;   // first vector index held in L
   const double one = 1.0, zero = 0.0, mone = -1.0;
   std::vector<double> hD;
   std::vector<long long> map;
@@ -538,35 +571,45 @@ void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_t
           THC_BLAS(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, ncand, ncand, npiv,
                                  &mone, w.pL[cur].p, ncand, w.pL[cur].p, ncand, &one, w.pS[scur].p, ncand));
         schur = true;
-        lbase = npiv;
       }
     }
     const long long max_j = std::min(block_dim, npts - npiv);
     if (schur)
-      w.pL[cur].alloc((size_t)(ncand * std::max<long long>(max_j, 1)));
+      w.pL[cur].alloc((size_t)(ncand * std::max<long long>(std::min<long long>(max_j, PIV_PANEL), 1)));
     else
       w.pL[cur].grow_keep((size_t)(ncand * (npiv + max_j)), C.stream);
-    if (schur) lbase = npiv;   // the block's vectors only
     // the state's done flag starts clear for every block
     st0.npiv = npiv;
     st0.done = 0;
     C.h2d(w.pstate.p, &st0, sizeof(st0));
     const unsigned gc = (unsigned)((ncand + 63) / 64);
-    const double *Sh = schur ? w.pS[scur].p : nullptr;
-    for (long long k = 0; k < max_j; ++k)
-      hipLaunchKernelGGL(k_thc_pivot_step, dim3(gc), dim3(1024), 0, C.stream, w.pX.p, ncand, nao, Sh, w.pL[cur].p,
-                         lbase, npiv + k, Dbuf[(dcur + k) & 1], Dbuf[(dcur + k + 1) & 1], w.pcand.p, w.ppiv.p, dst,
-                         thresh, thresh_red);
+    hipLaunchKernelGGL(k_thc_pivot_max, dim3(gc), dim3(64), 0, C.stream, Dbuf[dcur], ncand, Ebuf[0]);
+    if (schur) {
+      // panels of PIV_PANEL vectors, each taken off Shat by a DGEMM: a step
+      // then reads 64 vectors on average where it read half a block (2.4 us
+      // of memory at 9600 candidates and blocks of 500), and the DGEMMs' own
+      // operations are the same.  Once a step finds no pivot no candidate is
+      // left and Shat is not read again, whatever stands in the rest of L.
+      for (long long k0 = 0; k0 < max_j; k0 += PIV_PANEL) {
+        const long long kn = std::min<long long>(PIV_PANEL, max_j - k0);
+        for (long long k = k0; k < k0 + kn; ++k)
+          hipLaunchKernelGGL(k_thc_pivot_step<true>, dim3(gc), dim3(1024), 0, C.stream, w.pX.p, ncand, nao,
+                             w.pS[scur].p, w.pL[cur].p, npiv + k0, npiv + k, Dbuf[dcur], Ebuf[k & 1],
+                             Ebuf[(k + 1) & 1], w.pcand.p, w.ppiv.p, dst, thresh, thresh_red);
+        GI_HIP(hipGetLastError());
+        THC_BLAS(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, ncand, ncand, kn, &mone,
+                               w.pL[cur].p, ncand, w.pL[cur].p, ncand, &one, w.pS[scur].p, ncand));
+      }
+    } else {
+      for (long long k = 0; k < max_j; ++k)
+        hipLaunchKernelGGL(k_thc_pivot_step<false>, dim3(gc), dim3(1024), 0, C.stream, w.pX.p, ncand, nao, nullptr,
+                           w.pL[cur].p, 0LL, npiv + k, Dbuf[dcur], Ebuf[k & 1], Ebuf[(k + 1) & 1], w.pcand.p,
+                           w.ppiv.p, dst, thresh, thresh_red);
+    }
     GI_HIP(hipGetLastError());
     C.read(&st0, w.pstate.p, sizeof(st0));
-    const long long nblk = st0.npiv - npiv;
-    dcur = (int)((dcur + nblk) & 1);   // the buffer the block's last vector wrote
     npiv = st0.npiv;
     nred = st0.nred;
-    // Schur form: Shat -= L_blk L_blk^T
-    if (schur && nblk > 0)
-      THC_BLAS(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, ncand, ncand, nblk, &mone,
-                             w.pL[cur].p, ncand, w.pL[cur].p, ncand, &one, w.pS[scur].p, ncand));
     // compression: keep the candidates with D > thresh, in order
     hD.resize((size_t)ncand);
     C.read(hD.data(), Dbuf[dcur], sizeof(double) * ncand);

@@ -28,7 +28,7 @@ LIBS = ["-L/opt/rocm/lib", "-lrocsolver", "-lrocblas", "-Wl,-rpath,/opt/rocm/lib
 
 SOURCES = ["eri.hip", "chol.hip", "mo.hip", "grad.hip", "coul.hip", "coul6.hip", "coul7.hip", "split.hip", "crt.hip", "onee.hip", "aomap.hip", "thc.hip", "gi_tables.cpp",
            "gi_context.cpp", "sort.cpp", "capi.cpp"]
-HEADERS = ["gi_common.h", "gi_context.h", "md_kernel.h", "md4_kernel.h", "md_generic.h", "md_classes.inc", "grad_kernels.h", "coul_kernel.h", "crt.h", "coul_launch.h", "onee_kernels.h", "thc_kernels.h"]
+HEADERS = ["gi_common.h", "gi_context.h", "md_kernel.h", "md4_kernel.h", "md_generic.h", "md_classes.inc", "grad_kernels.h", "coul_kernel.h", "crt.h", "gi_wave.h", "coul_launch.h", "onee_kernels.h", "thc_kernels.h"]
 
 
 def _compile(src: str, incremental: bool) -> str:

@@ -19,7 +19,18 @@
 // are built together, all lanes over (quartet, entry) per recursion level.
 // Contracted pairs: X accumulates over ket primitives in registers; the
 // block of a contracted bra accumulates over its primitive pairs in place.
+//
+// What bounds it: vector instructions (six or seven per matrix instruction,
+// and FP64 matrix and vector instructions share their units) and the latency
+// of the recursion's levels at two to four waves per SIMD; the matrix
+// instructions take 15 to 30 % of the time, LDS 20 to 45 %.  Sum over the
+// classes, one after the other: (H2O)12, 900 AOs, uncontracted 35.0 -> 30.2 ms,
+// (H2O)5, 375 AOs, contracted 216 -> 135 ms, from the recursion by levels at
+// LDS latency (md4_rtable), Boys passes over several primitive steps, and
+// stage-1 reads ahead of their instructions.  Tried without gain: records, row
+// tables and row groups of all bra pairs of a tile fetched ahead.
 #pragma once
+#include <type_traits>
 #include "md_kernel.h"
 
 namespace gi {
@@ -79,6 +90,11 @@ __device__ __forceinline__ double buf_ld(__amdgpu_buffer_rsrc_t r, unsigned voff
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
 }
 
+// reads of the R table ahead of the stage-1 instructions
+#ifndef MD4_S1D
+#define MD4_S1D 8
+#endif
+
 // bra pairs per tile (rows of one column tile handled by one wavefront)
 #ifndef MD4_NB
 #define MD4_NB 4
@@ -119,25 +135,131 @@ __device__ __forceinline__ void md4_boys(const PrimRec &PB, const PrimRec &PK, d
   PQ[2] = PQz;
 }
 
+// Orders the LDS accesses of a one-wave workgroup: a wave's LDS instructions
+// execute in order, so only the compiler has to keep the order (a workgroup
+// barrier would wait for every write to return before the next read).
+__device__ __forceinline__ void m4_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_wave_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// R table of one quartet by LPQ lanes (sub = 0 .. LPQ - 1), from its scaled
+// Boys values F[0..L] and P - Q: the recursion
+//   R^(n)_{tuv} = coef R^(n+1)_{i2} + PQ_dir R^(n+1)_{i1},
+// levels L-1 .. 1 in the ping-pong tables Ra (odd levels) and Rb (even), level
+// 0 into the dense table.  A lane's entries and their codes are the same at
+// every level, so they are decoded once, a level's operands are read together,
+// and the levels follow each other at LDS latency.  With run-time lane counts,
+// codes fetched per entry and a barrier per level the recursion was two thirds
+// of the time of the middle orders.  PACKED: level 0 stays packed, in Rb.
+template <int L, int LPQ, bool PACKED>
+__device__ __forceinline__ void md4_rtable(double *Rd, double *Ra, double *Rb, const double *F, const double *PQ,
+                                           const int *s_rrec, const unsigned short *s_dix, int sub, bool act) {
+  constexpr int NHL = nherm(L), NJ = (NHL + LPQ - 1) / LPQ;
+  m4_fence();   // Boys values written; earlier readers of the tables are ahead in the queue
+  if (act) {
+    if constexpr (L == 0) {
+      if (sub == 0) Rd[0] = F[0];
+    } else {
+      const double pqx = PQ[0], pqy = PQ[1], pqz = PQ[2];
+      // decoded once where few (byte offsets of i1 and i2, coefficient, PQ_dir),
+      // at each level from the packed codes where the decoded ones would cost
+      // occupancy
+      constexpr bool KEEP = NJ <= 8;
+      unsigned oo[NJ];
+      float cf[NJ];
+      double pd[NJ];
+      auto decode = [&](int rec, unsigned &o, float &c, double &p) {
+        const int dir = (rec >> 22) & 3;
+        o = 8u * (rec & 0x7ff) | (8u * ((rec >> 11) & 0x7ff)) << 16;
+        c = (float)(rec >> 24);
+        p = dir == 0 ? pqx : (dir == 1 ? pqy : pqz);
+      };
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int idx = sub + LPQ * j, rec = s_rrec[idx < NHL ? idx : 0];
+        if (KEEP) decode(rec, oo[j], cf[j], pd[j]);
+        else oo[j] = rec;
+      }
+      double *const T[2] = {Rb, Ra};   // by level parity
+      if (sub == 0) T[L % 2][0] = F[L];
+#pragma unroll
+      for (int n = L - 1; n >= 0; --n) {
+        m4_fence();
+        const int cnt = nherm(L - n);
+        const double *prv = T[(n + 1) % 2];
+        double *cur = T[n % 2];
+        const double f = F[n];
+        // eight entries of a lane at a time: their reads go out together
+#pragma unroll
+        for (int j0 = 0; j0 < NJ; j0 += 8) {
+          if (LPQ * j0 >= cnt) break;
+          double r[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int j = j0 + i;
+            if (j < NJ && LPQ * j < cnt) {
+              unsigned o = oo[j];
+              float c = cf[j];
+              double p = pd[j];
+              if (!KEEP) {
+                int rec = (int)oo[j];
+                asm volatile("" : "+v"(rec));   // decoded here, not hoisted
+                decode(rec, o, c, p);
+              }
+              const double p1 = *(const double *)((const char *)prv + (o & 0xffffu));
+              const double p2 = *(const double *)((const char *)prv + (o >> 16));
+              r[i] = fma((double)c, p2, p * p1);
+            }
+          }
+          if (j0 == 0 && sub == 0) r[0] = f;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            const int j = j0 + i;
+            if (j < NJ && LPQ * j < cnt) {
+              if (LPQ * (j + 1) <= cnt || sub + LPQ * j < cnt) {
+                if (n == 0 && !PACKED) Rd[s_dix[sub + LPQ * j]] = r[i];
+                else cur[sub + LPQ * j] = r[i];
+              }
+            }
+          }
+          if (!KEEP) asm volatile("" ::: "memory");
+        }
+      }
+    }
+  }
+  m4_fence();
+}
+
 // PLAIN: every pair of the launch has one primitive pair (uncontracted), so the
 // kernel omits the primitive loops
-// Waves per SIMD asked of the compiler for the classes whose register count
-// lay a few registers above the next occupancy step: it then keeps the MFMA
-// accumulators in VGPRs instead of AGPRs and reaches the step with no
-// scratch.  Measured per class on the (H2O)16 builds:
-//   uncontracted, three waves: (1,6) -21 %, (2,5) -12 %, (2,6) -7 %, (5,2) -6 %,
-//     (4,4) -2 %; four waves for (2,3), (3,2), (3,4), (4,0), (4,1) or three for
-//     (0,6), (3,5), (5,0) changed nothing or slowed them ((3,4) +15 %);
+// Waves per SIMD asked of the compiler: two keeps the MFMA accumulators in
+// VGPRs (left alone it puts them in AGPRs for most classes, which cost (5,6)
+// 21 %, (6,5) and (5,3) 15 %), more where the register count lay a few
+// registers above the next step.  Measured per class, (H2O)12 uncontracted and
+// (H2O)5 contracted, against the compiler's own choice:
+//   uncontracted, three waves: (2,4), (3,3) -15 %, (1,6) -21 %, (2,5), (2,6),
+//     (5,2) -6 to -12 %, (4,2..4) -2 to -8 %; four waves for (2,3), (3,2),
+//     (3,4), (4,0), (4,1) or three for (0,6), (5,0), (5,1) changed nothing or
+//     slowed them;
 //   contracted, four waves for (0,3), (1,3), (2,0..2), three for (0,4), (2,3),
-//     (2,4), (3,2), (3,4), (4,2), (4,3): 8 to 17 % each, none slower.
-// Higher orders spill under either request.
+//     (2,4), (3,2), (3,4), (4,2), (4,3): 8 to 17 % each; two for (3,1), (4,6),
+//     (5,5), (5,6), (6,4), (6,5): 7 to 25 %.  Two slows the others by 2 to 9 %.
+// (6,6) spills under either request.
 __host__ __device__ constexpr int md4_min_waves(int E, int F, bool plain) {
-  if (plain) return ((E == 1 && F == 6) || (E == 2 && F >= 5) || (E == 4 && F == 4) || (E == 5 && F == 2)) ? 3 : 1;
+  if (E == 6 && F == 6) return 1;
+  if (plain)
+    return ((E == 1 && F == 6) || (E == 2 && F >= 4) || (E == 3 && F == 3) || (E == 4 && F >= 2 && F <= 4) ||
+            (E == 5 && F == 2))
+               ? 3
+               : 2;
   return ((E == 0 && F == 3) || (E == 1 && F == 3) || (E == 2 && F <= 2)) ? 4
          : ((E == 0 && F == 4) || (E == 2 && (F == 3 || F == 4)) || (E == 3 && (F == 2 || F == 4)) ||
             (E == 4 && (F == 2 || F == 3)))
              ? 3
-             : 1;
+         : ((E == 3 && F == 1) || (E == 4 && F == 6) || (E == 5 && F >= 5) || (E == 6 && F >= 4)) ? 2
+                                                                                                  : 1;
 }
 
 template <int E, int F, bool PLAIN>
@@ -148,8 +270,12 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
   constexpr int DS = S::DS, QM = S::QM, NL1 = S::NL1;
   __shared__ double s_Rd[QM][DS];              // level-0 R tables, dense
   __shared__ double s_Rp[2][QM][NL1];          // levels >= 1, packed (ping-pong)
-  __shared__ double s_F[M4_NB][QM][L + 1];     // scaled Boys values per (bra pair, quartet)
-  __shared__ double s_PQ[M4_NB][QM][4];        // P - Q per (bra pair, quartet)
+  // quartets whose Boys values are evaluated in one pass, a lane each: the
+  // tile's (bra pair, ket pair) quartets, or the primitive quartets of
+  // consecutive steps (fewer of them where LDS would cost occupancy)
+  constexpr int BL = PLAIN ? M4_NB * QM : (QM == 1 ? 16 : (md4_min_waves(E, F, PLAIN) >= 4 ? 32 : 64));
+  __shared__ double s_F[BL][L + 1];            // scaled Boys values per quartet
+  __shared__ double s_PQ[BL][4];               // P - Q per quartet
   __shared__ int s_rrec[NHL];
   __shared__ unsigned short s_dix[NHL];        // dense offset of packed index
   __shared__ int s_hoff[NHG * 4];              // dense offset of h (0 for padding)
@@ -204,39 +330,18 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
   const long long nrb = (A.nrows + nbr - 1) / nbr;
   const long long ntiles = nrb * nct;
 
-  // R tables of the nq quartets of bra pair b (Boys values in s_F[b], s_PQ[b]):
-  // the recursion R^(n)_{tuv} = coef R^(n+1)_{i2} + PQ_dir R^(n+1)_{i1},
-  // levels L-1 .. 0, lpq lanes per quartet; level 0 into the dense tables
-  auto build_r = [&](int b, int nq, unsigned actmask) {
-    const int lpq = nq <= 1 ? 64 : (nq == 2 ? 32 : 16);
-    const int ql = lane / lpq, sub = lane - ql * lpq;
-    const bool act = ql < nq && ((actmask >> ql) & 1u);
-    __syncthreads();   // Boys values written; earlier readers of the tables are done
-    if (act && L > 0 && sub == 0) s_Rp[L % 2][ql][0] = s_F[b][ql][L];
-    if (act && L == 0 && sub == 0) s_Rd[ql][0] = s_F[b][ql][0];
-#pragma unroll
-    for (int n = L - 1; n >= 0; --n) {
-      __syncthreads();
-      const int cnt = nherm(L - n);
-      if (act) {
-        const double *prv = s_Rp[(n + 1) % 2][ql];
-        for (int idx = sub; idx < cnt; idx += lpq) {
-          double r;
-          if (idx == 0) {
-            r = s_F[b][ql][n];
-          } else {
-            const int rec = s_rrec[idx];
-            const int i1 = rec & 0x7ff, i2 = (rec >> 11) & 0x7ff, dir = (rec >> 22) & 3, coef = rec >> 24;
-            r = (double)coef * prv[i2] + s_PQ[b][ql][dir] * prv[i1];
-          }
-          if (n == 0)
-            s_Rd[ql][s_dix[idx]] = r;
-          else
-            s_Rp[n % 2][ql][idx] = r;
-        }
-      }
-    }
-    __syncthreads();
+  // R tables of the nq quartets whose Boys values start at f0: 64, 32 or 16
+  // lanes per quartet
+  auto build_r = [&](int f0, int nq, unsigned actmask) {
+    auto build = [&](auto lpq) {
+      constexpr int LPQ = decltype(lpq)::value;
+      const int ql = lane / LPQ, sub = lane % LPQ, q = ql < QM ? ql : 0;
+      md4_rtable<L, LPQ, false>(s_Rd[q], s_Rp[1][q], s_Rp[0][q], s_F[f0 + (ql < nq ? ql : 0)], s_PQ[f0 + (ql < nq ? ql : 0)],
+                         s_rrec, s_dix, sub, ql < nq && ((actmask >> ql) & 1u));
+    };
+    if (QM == 1 || nq == 1) build(std::integral_constant<int, 64>{});
+    else if (QM == 2 || nq == 2) build(std::integral_constant<int, 32>{});
+    else build(std::integral_constant<int, 16>{});
   };
 
   for (long long t = v0; t < ntiles; t += G) {
@@ -260,10 +365,11 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
     // each waiting behind a branch
     double eb[KSF];
     auto load_eb = [&](int kp) {
+      // the tables of a pair's primitives follow each other (eri_run), so their
+      // addresses need no primitive record
       const bool kval = cval && kp < CD.nprim;
       const int kpc = kp < CD.nprim ? kp : CD.nprim - 1;
-      const PrimRec PKm = kpc == 0 ? first_prim(CD) : A.prim[CD.prim0 + kpc];
-      const double *etk = A.et + PKm.et;
+      const double *etk = A.et + CD.et + (long long)(kpc * (NHF * ldk));
 #pragma unroll
       for (int kg = 0; kg < KSF; ++kg) {
         const int k = 4 * kg + lq;
@@ -279,25 +385,41 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
     // stage 1: X(h, c) += sum_k R_{h+k} B(k, c) from the dense table of this
     // lane's slot; k step kg updates NHG independent accumulators (the step's
     // offset passes through an empty asm statement so that the NHG addresses
-    // are formed in the step instead of all NHG x KSF hoisted into registers)
+    // are formed in the step instead of all NHG x KSF hoisted into registers).
+    // The reads run S1D instructions ahead: left to the compiler every
+    // instruction waited for its own read, some 130 cycles in place of 16.
     double X[NHG];
     auto stage1 = [&]() {
       const double *Rq = s_Rd[myrt];
+      // (two more places than reads in flight, so that a read does not wait for
+      // the instruction that used its place last)
+      constexpr int N = KSF * NHG, S1D = imin(MD4_S1D, N), NS = S1D + 2;
+      double rv[NS];
+      int ko = 0;
+      auto rd = [&](int i) {
+        if (i % NHG == 0) {
+          ko = koff[i / NHG];
+          asm volatile("" : "+v"(ko));
+        }
+        rv[i % NS] = (Rq + ko)[hoff[i % NHG]];
+      };
 #pragma unroll
-      for (int kg = 0; kg < KSF; ++kg) {
-        int ko = koff[kg];
-        asm volatile("" : "+v"(ko));
-        const double *Rk = Rq + ko;
+      for (int i = 0; i < S1D; ++i) rd(i);
 #pragma unroll
-        for (int hg = 0; hg < NHG; ++hg) X[hg] = __builtin_amdgcn_mfma_f64_4x4x4f64(Rk[hoff[hg]], eb[kg], X[hg], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      for (int kg = 0; kg < KSF; ++kg)
+#pragma unroll
+        for (int hg = 0; hg < NHG; ++hg) {
+          const int i = kg * NHG + hg;
+          __builtin_amdgcn_sched_barrier(0);
+          if (i + S1D < N) rd(i + S1D);
+          X[hg] = __builtin_amdgcn_mfma_f64_4x4x4f64(rv[i % NS], eb[kg], X[hg], 0, 0, 0);
+        }
     };
     // bra rows of RB: byte offset of each row's full-block index
     auto fill_rows = [&](const QRec &RB) {
       for (int r = lane; r < RB.nrow; r += 64) s_frow[r] = 8u * (unsigned)pair_full(RB, A.sel, r);
       if (lane < 4) s_frow[RB.nrow + lane] = 0u;   // padding rows of the last row group
-      __syncthreads();
+      m4_fence();
     };
     // stage 2 for one bra primitive pair: V(r, c) = sum_h ET_bra(h, r) X(h, c),
     // four bra rows per step (the A operand's row 4 rg + li); the table of h step
@@ -327,7 +449,7 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
     // two accumulator chains (even and odd h steps)
     auto stage2 = [&](const QRec &RB, bool accumulate) {
       const int nr = RB.nrow;
-      double *const out = A.out + RB.off + CD.off;
+      double *d = A.out + RB.off + CD.off + rs * lq + cs * c;
       const int nrg = (nr + 3) / 4;
       for (int rg = 0; rg < nrg; ++rg) {
         double e[NHG];
@@ -343,11 +465,8 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
           else
             v0 = __builtin_amdgcn_mfma_f64_4x4x4f64(e[hg], X[hg], v0, 0, 0, 0);
         }
-        const int ro = 4 * rg + lq;
-        if (cval && ro < nr) {
-          double *d = out + rs * ro + cs * c;
-          *d = accumulate ? *d + (v0 + v1) : v0 + v1;
-        }
+        if (cval && 4 * rg + lq < nr) *d = accumulate ? *d + (v0 + v1) : v0 + v1;
+        d += 4 * rs;
       }
     };
 
@@ -355,19 +474,19 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
       // uncontracted tile: one Boys pass for every (bra pair, ket pair)
       // quartet of the tile, then per bra pair the R tables and both stages
       load_eb(0);
-      __syncthreads();   // earlier readers of s_F / s_PQ are done
+      m4_fence();   // earlier readers of s_F / s_PQ are done
       if (lane < nb * nq) {
         const int b = lane / nq, q = lane - b * nq;
         const QRec RB = A.rrec[ir0 + b];
         const QRec CQ = A.crec[pick4(T.jq, q)];
-        md4_boys<L>(first_prim(RB), first_prim(CQ), A.kappa, A.boys, s_F[b][q], s_PQ[b][q]);
+        md4_boys<L>(first_prim(RB), first_prim(CQ), A.kappa, A.boys, s_F[lane], s_PQ[lane]);
       }
       for (int b = 0; b < nb; ++b) {
         const QRec RB = load_rec_uniform(rrec + ir0 + b);
         fill_rows(RB);
         s2_open(RB, A.et + RB.et);
         load_rows(0);
-        build_r(b, nq, 0xfu);
+        build_r(b * nq, nq, 0xfu);
 #pragma unroll
         for (int hg = 0; hg < NHG; ++hg) X[hg] = 0.0;
         stage1();
@@ -376,39 +495,62 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
     } else {
       // contracted pairs: per bra pair and bra primitive pair, X summed over
       // the ket primitive pairs; the block accumulates over bra primitives.
-      // The Boys values of up to M4_NB ket primitive steps are evaluated in
-      // one pass (one lane per step and quartet) before their R tables.
-      int maxnp = 1;
-      for (int qq = 0; qq < nq; ++qq) maxnp = imax(maxnp, A.crec[pick4(T.jq, qq)].nprim);
+      // Steps (bra pair, bra primitive, ket primitive) are numbered through the
+      // tile, and the Boys values of as many steps as there are lanes are
+      // evaluated in one pass: it is a chain of some 400 dependent operations,
+      // and a pass of at most four steps left most of its lanes idle.
+      int npk[4], nprb[M4_NB], maxnp = 1, tot = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        npk[q] = q < nq ? __builtin_amdgcn_readfirstlane(A.crec[T.jq[q]].nprim) : 0;
+        maxnp = imax(maxnp, npk[q]);
+      }
+#pragma unroll
+      for (int b = 0; b < M4_NB; ++b) {
+        nprb[b] = b < nb ? __builtin_amdgcn_readfirstlane(rrec[ir0 + b].nprim) : 0;
+        tot += nprb[b];
+      }
+      tot *= maxnp;
+      const int spc = imin(64, BL) / nq;   // steps per Boys pass
+      int step = 0, chunk = -spc;
       for (int b = 0; b < nb; ++b) {
         const QRec RB = load_rec_uniform(rrec + ir0 + b);
         fill_rows(RB);
         for (int bp = 0; bp < RB.nprim; ++bp) {
-          const PrimRec PB = bp == 0 ? first_prim(RB) : A.prim[RB.prim0 + bp];
-          s2_open(RB, A.et + PB.et);
+          s2_open(RB, A.et + RB.et + (long long)(bp * (NHE * RB.n0 * RB.n1)));
           load_rows(0);
 #pragma unroll
           for (int hg = 0; hg < NHG; ++hg) X[hg] = 0.0;
-          for (int kp0 = 0; kp0 < maxnp; kp0 += M4_NB) {
-            const int nkk = imin(M4_NB, maxnp - kp0);
-            __syncthreads();   // earlier readers of the R tables and s_F are done
-            if (lane < nkk * nq) {
-              const int kk = lane / nq, q = lane - kk * nq, kp = kp0 + kk;
-              const QRec CQ = A.crec[pick4(T.jq, q)];
-              if (kp < CQ.nprim) {
-                const PrimRec PK = kp == 0 ? first_prim(CQ) : A.prim[CQ.prim0 + kp];
-                md4_boys<L>(PB, PK, A.kappa, A.boys, s_F[kk][q], s_PQ[kk][q]);
+          for (int kp = 0; kp < maxnp; ++kp, ++step) {
+            if (step >= chunk + spc) {
+              chunk = step;
+              m4_fence();   // earlier readers of s_F are done
+              const int si = lane / nq, q = lane - si * nq;
+              int r = step + si;
+              if (si < spc && r < tot) {
+                int bb = 0;
+#pragma unroll
+                for (int k = 0; k + 1 < M4_NB; ++k)
+                  if (bb == k && r >= nprb[k] * maxnp) {
+                    r -= nprb[k] * maxnp;
+                    bb = k + 1;
+                  }
+                const int bpp = r / maxnp, kpp = r - bpp * maxnp;
+                const QRec CQ = A.crec[pick4(T.jq, q)];
+                if (kpp < CQ.nprim) {
+                  const QRec RQ = A.rrec[ir0 + bb];
+                  const PrimRec PB = bpp == 0 ? first_prim(RQ) : A.prim[RQ.prim0 + bpp];
+                  const PrimRec PK = kpp == 0 ? first_prim(CQ) : A.prim[CQ.prim0 + kpp];
+                  md4_boys<L>(PB, PK, A.kappa, A.boys, s_F[lane], s_PQ[lane]);
+                }
               }
             }
-            for (int kk = 0; kk < nkk; ++kk) {
-              const int kp = kp0 + kk;
-              unsigned act = 0;
-              for (int qq = 0; qq < nq; ++qq)
-                if (kp < A.crec[pick4(T.jq, qq)].nprim) act |= 1u << qq;
-              build_r(kk, nq, act);
-              load_eb(kp);
-              stage1();
-            }
+            unsigned act = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) act |= kp < npk[q] ? 1u << q : 0u;
+            load_eb(kp);   // on its way during the recursion
+            build_r((step - chunk) * nq, nq, act);
+            stage1();
           }
           stage2(RB, bp > 0);
         }
@@ -431,15 +573,22 @@ md4_kernel(MdArgs A, const ColTile *__restrict__ ctiles, long long nct, const QR
 // evaluated them and reach the recursion lanes by cross-lane reads.
 constexpr int M4S_NK = 16;
 
+// (as the compiler would choose, but without AGPRs and without the decoded
+// recursion codes' registers: (6,0) 3.6 -> 2.2 ms and (0,6) 3.2 -> 1.9 ms per
+// contracted (H2O)5 build, with four primitive steps per Boys pass)
+__host__ __device__ constexpr int md4s_min_waves(int E, bool plain) {
+  return E == 6 ? 2 : (E == 5 ? (plain ? 3 : 2) : (E == 4 ? 3 : 4));
+}
+
 template <int E, bool PLAIN>
-__global__ void __launch_bounds__(64) MD4_ATTR md4s_kernel(MdArgs A, const QRec *__restrict__ rrec) {
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(md4s_min_waves(E, PLAIN)))) MD4_ATTR
+md4s_kernel(MdArgs A, const QRec *__restrict__ rrec) {
   constexpr int L = E, NHE = nherm(E), NHG = (NHE + 3) / 4;
   constexpr int NL1 = L >= 1 ? nherm(L - 1) : 1;
   constexpr int SB = NHE | 1, SA = NL1 | 1;   // odd row strides (LDS banks)
   constexpr int NRMAX = nab_max(E);
   __shared__ double s_Rb[M4S_NK * SB];        // even levels, level 0 last
   __shared__ double s_Ra[M4S_NK * SA];        // odd levels
-  __shared__ double s_pq[M4S_NK][4];          // P - Q of the bra pair's quartets
   __shared__ int s_rrec[NHE];
   __shared__ unsigned s_frow[NRMAX + 4];
 
@@ -469,37 +618,13 @@ __global__ void __launch_bounds__(64) MD4_ATTR md4s_kernel(MdArgs A, const QRec 
   // R tables of the sixteen quartets whose Boys values sit in lanes
   // src0 .. src0 + 15: lanes 4 j .. 4 j + 3 recurse quartet j
   auto build_r = [&](int src0) {
-    const int j = lane >> 2, sub = lane & 3;
-    const int src = src0 + j;
-    const double px_ = __shfl(PQq[0], src), py_ = __shfl(PQq[1], src), pz_ = __shfl(PQq[2], src);
-    const double ftop = __shfl(Fq[L], src);
-    __syncthreads();   // earlier readers of the tables are done
-    if (sub == 0) {
-      s_pq[j][0] = px_;
-      s_pq[j][1] = py_;
-      s_pq[j][2] = pz_;
-      ((L & 1) ? s_Ra + j * SA : s_Rb + j * SB)[0] = ftop;
-    }
+    const int j = lane >> 2, src = src0 + j;
+    double F[L + 1], PQ[3];
 #pragma unroll
-    for (int n = L - 1; n >= 0; --n) {
-      const double fn = __shfl(Fq[n], src);
-      __syncthreads();
-      const int cnt = nherm(L - n);
-      const double *prv = ((n + 1) & 1) ? s_Ra + j * SA : s_Rb + j * SB;
-      double *cur = (n & 1) ? s_Ra + j * SA : s_Rb + j * SB;
-      for (int idx = sub; idx < cnt; idx += 4) {
-        double r;
-        if (idx == 0) {
-          r = fn;
-        } else {
-          const int rec = s_rrec[idx];
-          const int i1 = rec & 0x7ff, i2 = (rec >> 11) & 0x7ff, dir = (rec >> 22) & 3, coef = rec >> 24;
-          r = (double)coef * prv[i2] + s_pq[j][dir] * prv[i1];
-        }
-        cur[idx] = r;
-      }
-    }
-    __syncthreads();
+    for (int n = 0; n <= L; ++n) F[n] = __shfl(Fq[n], src);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) PQ[d] = __shfl(PQq[d], src);
+    md4_rtable<L, 4, true>(s_Rb + j * SB, s_Ra + j * SA, s_Rb + j * SB, F, PQ, s_rrec, nullptr, lane & 3, true);
   };
   // stage 1: X(h, c) (+)= R_h ET_ket(c) for this lane's h = 4 hg + lq, c = col
   double X[NHG];
@@ -516,7 +641,7 @@ __global__ void __launch_bounds__(64) MD4_ATTR md4s_kernel(MdArgs A, const QRec 
   auto fill_rows = [&](const QRec &RB) {
     for (int r = lane; r < RB.nrow; r += 64) s_frow[r] = 8u * (unsigned)pair_full(RB, A.sel, r);
     if (lane < 4) s_frow[RB.nrow + lane] = 0u;
-    __syncthreads();
+    m4_fence();
   };
   // stage 2 as in md4_kernel (first row group loaded ahead): V(r, c) =
   // sum_h ET_bra(h, r) X(h, c), column c of this lane the single column of
@@ -597,32 +722,31 @@ __global__ void __launch_bounds__(64) MD4_ATTR md4s_kernel(MdArgs A, const QRec 
       }
     } else {
       // contracted pairs: per bra pair and bra primitive pair, X summed over
-      // the ket primitive pairs (lanes 0 .. 15 evaluate the Boys values of the
-      // sixteen quartets of one primitive step)
+      // the ket primitive pairs.  Steps (bra primitive, ket primitive) of a bra
+      // pair are numbered, and one Boys pass serves four of them, lanes
+      // 16 s .. 16 s + 15 the sixteen quartets of step s.
       int maxnp = 1;
       for (int j = 0; j < nk; ++j) maxnp = imax(maxnp, A.crec[jc0 + j].nprim);
+      maxnp = __builtin_amdgcn_readfirstlane(maxnp);
       for (int b = 0; b < nb; ++b) {
         const QRec RB = load_rec_uniform(rrec + ir0 + b);
         fill_rows(RB);
+        int step = 0;
         for (int bp = 0; bp < RB.nprim; ++bp) {
-          const PrimRec PB = bp == 0 ? first_prim(RB) : A.prim[RB.prim0 + bp];
-          s2_open(RB, A.et + PB.et);
+          s2_open(RB, A.et + RB.et + (long long)(bp * (NHE * RB.n0 * RB.n1)));
           load_rows(0);
-          for (int kp = 0; kp < maxnp; ++kp) {
-            clear_boys();
-            if (lane < nk) {
-              const QRec CQ = A.crec[jc0 + lane];
-              if (kp < CQ.nprim) {
-                const PrimRec PK = kp == 0 ? first_prim(CQ) : A.prim[CQ.prim0 + kp];
+          for (int kp = 0; kp < maxnp; ++kp, ++step) {
+            if ((step & 3) == 0) {
+              const int st = step + lq, bpp = st / maxnp, kpp = st - bpp * maxnp;
+              clear_boys();
+              if (cval && bpp < RB.nprim && kpp < CD.nprim) {
+                const PrimRec PB = bpp == 0 ? first_prim(RB) : A.prim[RB.prim0 + bpp];
+                const PrimRec PK = kpp == 0 ? first_prim(CD) : A.prim[CD.prim0 + kpp];
                 md4_boys<L>(PB, PK, A.kappa, A.boys, Fq, PQq);
               }
             }
-            build_r(0);
-            double etv = 0.0;
-            if (cval && kp < CD.nprim) {
-              const PrimRec PK = kp == 0 ? first_prim(CD) : A.prim[CD.prim0 + kp];
-              etv = A.et[PK.et + fc];
-            }
+            const double etv = cval && kp < CD.nprim ? A.et[CD.et + (long long)(kp * (CD.n0 * CD.n1)) + fc] : 0.0;
+            build_r(16 * (step & 3));
             stage1(etv, kp > 0);
           }
           stage2(RB, outc, cval, bp > 0);

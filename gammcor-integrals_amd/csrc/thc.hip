@@ -149,6 +149,8 @@ __global__ void __launch_bounds__(256) k_thc_pair_products(const double *__restr
 //   Schur        Shat(:,h) - sum over the block's vectors only, where Shat is
 //                S less the earlier blocks' vectors, kept explicitly (one DGEMM
 //                per block updates it): reads one column and the block per pivot.
+//                Shat is symmetric and kept in block columns of PIV_COLS from
+//                their diagonal block down (thc_lower_update).
 // The library uses the Schur form when the candidates' Shat fits the
 // thc_schur_mb budget and the on-the-fly form before that.
 struct PivotState {
@@ -201,6 +203,10 @@ __global__ void __launch_bounds__(64) k_thc_pivot_max(const double *__restrict__
 // here, and about 2.5 us between two launches.  Pruning 9600 points (6000
 // pivots, 600 AOs): 92 -> 57 ms.
 constexpr int PIV_PANEL = 128;   // Schur form: vectors kept outside Shat
+// Schur form: columns of a block column of Shat.  A DGEMM of the whole square
+// updates every element twice (43 of 378 us, 16.3 of 54 ms, when 9600 points are
+// pruned); narrower blocks save more but leave the last ones too few tiles.
+constexpr int PIV_COLS = 1024;
 template <bool SCHUR>
 __global__ void __launch_bounds__(1024) k_thc_pivot_step(const double *__restrict__ X, long long ncand,
                                                          long long nao, const double *__restrict__ Sh,
@@ -247,7 +253,8 @@ __global__ void __launch_bounds__(1024) k_thc_pivot_step(const double *__restric
   if constexpr (SCHUR) {
     const int j = w + 16 * (lane & (NJ - 1));
     const double lh = j < kl ? L[h + ncand * j] : 0.0;   // lane i: the pivot's element of this wave's term i
-    if (w == 0 && ok) col = Sh[g + ncand * h];
+    // a pivot's row of the earlier block columns stands in for its column there
+    if (w == 0 && ok) col = g >= h / PIV_COLS * PIV_COLS ? Sh[g + ncand * h] : Sh[h + ncand * g];
 #pragma unroll
     for (int i = 0; i < NJ; ++i) c += lg[i] * read_lane(lh, i);
   } else if (ok) {
@@ -275,14 +282,20 @@ __global__ void __launch_bounds__(1024) k_thc_pivot_step(const double *__restric
   }
 }
 
-// Shat(i, j) of the kept candidates: out(i, j) = in(map[i], map[j])
+// Shat(i, j) of the kept candidates, out(i, j) = in(map[i], map[j]), from the
+// diagonal blocks down; map ascends, and what a new diagonal block has above
+// its diagonal is read below the old one
 __global__ void __launch_bounds__(256) k_thc_gather_square(const long long *__restrict__ map, long long nnew,
                                                            long long nold, const double *__restrict__ in,
                                                            double *__restrict__ out) {
   const long long i = blockIdx.x * 256LL + threadIdx.x;
   if (i >= nnew) return;
   const long long si = map[i];
-  for (long long j = blockIdx.y; j < nnew; j += gridDim.y) out[i + nnew * j] = in[si + nold * map[j]];
+  for (long long j = blockIdx.y; j < nnew; j += gridDim.y) {
+    if (i < j / PIV_COLS * PIV_COLS) continue;
+    const long long sj = map[j];
+    out[i + nnew * j] = i < j ? in[sj + nold * si] : in[si + nold * sj];
+  }
 }
 
 // compression (thc_Chol_Compress, :1067-1127): candidate rows map[i] of the
@@ -515,6 +528,14 @@ void thc_rkab(Context &C, const double *dX, long long ldx, long long npts, const
   C.wait();
 }
 
+// Shat -= L L^T (kn vectors), block columns from their diagonal block down
+static void thc_lower_update(Context &C, long long n, long long kn, const double *L, double *S) {
+  const double one = 1.0, mone = -1.0;
+  for (long long c = 0; c < n; c += PIV_COLS)
+    THC_BLAS(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, n - c,
+                           std::min<long long>(PIV_COLS, n - c), kn, &mone, L + c, n, L + c, n, &one, S + c + n * c, n));
+}
+
 // thc_Chol_Pivots (TensorHypercontraction.f90:772-968) on the device: blocks of
 // at most block_dim pivots, one launch per step (a step after the last pivot
 // exits at once), one synchronization per block for the compression.  dxyz: the parent points (3, npts), device.
@@ -549,7 +570,7 @@ void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_t
   PivotState *dst = (PivotState *)w.pstate.p;
   int cur = 0, scur = 0;
   bool converged = false, schur = false;
-  const double one = 1.0, zero = 0.0, mone = -1.0;
+  const double one = 1.0, zero = 0.0;
   std::vector<double> hD;
   std::vector<long long> map;
   for (long long it = 0; it < max_iters; ++it) {
@@ -568,8 +589,7 @@ void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_t
                            w.pS[scur].p, ncand, ncand);
         GI_HIP(hipGetLastError());
         if (npiv > 0)
-          THC_BLAS(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, ncand, ncand, npiv,
-                                 &mone, w.pL[cur].p, ncand, w.pL[cur].p, ncand, &one, w.pS[scur].p, ncand));
+          thc_lower_update(C, ncand, npiv, w.pL[cur].p, w.pS[scur].p);
         schur = true;
       }
     }
@@ -597,8 +617,7 @@ void thc_grid_pivots(Context &C, const double *dxyz, long long npts, double qr_t
                              w.pS[scur].p, w.pL[cur].p, npiv + k0, npiv + k, Dbuf[dcur], Ebuf[k & 1],
                              Ebuf[(k + 1) & 1], w.pcand.p, w.ppiv.p, dst, thresh, thresh_red);
         GI_HIP(hipGetLastError());
-        THC_BLAS(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_transpose, ncand, ncand, kn, &mone,
-                               w.pL[cur].p, ncand, w.pL[cur].p, ncand, &one, w.pS[scur].p, ncand));
+        thc_lower_update(C, ncand, kn, w.pL[cur].p, w.pS[scur].p);
       }
     } else {
       for (long long k = 0; k < max_j; ++k)

@@ -40,3 +40,13 @@ def test_candidate_counts(case, n, schur_mb):
     finally:
         c.set_option("thc_schur_mb", 24576)
     assert gred == nred and np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("n", [1023, 1025, 2160])
+def test_block_columns(case, n):
+    """Candidates around the 1024 columns of a block column of the Schur form."""
+    c, b, _ = case
+    pts = systems.atom_centred_points(b, radii=(0.2, 0.5, 0.9, 1.5, 2.4, 3.6), ndir=120, seed=8)[:n]
+    ref, nred = thc_oracle.grid_pivots(b, pts, 1e-3, 1e-2, 200)
+    got, gred = c.thc_grid_pivots(pts, 1e-3, 1e-2, 200)
+    assert gred == nred and np.array_equal(got, ref)

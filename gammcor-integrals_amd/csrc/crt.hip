@@ -322,28 +322,46 @@ __global__ void __launch_bounds__(256, 1) k_crt_gemm(CrtGemm G, const CrtConst *
   // residues to bytes through LDS ([column][row], rows padded by four bytes), then whole rows of R
   constexpr int LD = CRT_T / 4 + 1;   // dwords
   int *t = (int *)&st[0][0][0];
-  const int m = (int)K->m[mod];
+  // The quotient's low bits stand in the low bits of x / m + 1.5 2^23, and the
+  // byte of x - m q needs no others.  Below 2^22 the float of x is exact and
+  // the quotient off from rounding by under 0.001 (the limit is 0.0019: m = 255
+  // must leave |x - m q| <= 128); larger sums, which need a long k, are first
+  // brought below 2 m.  Three operations an element, with two integer
+  // multiplications and two roundings in their place the ends of the tiles took
+  // as long as 18 stages.
+  const unsigned m = (unsigned)(int)K->m[mod], nm = 0x1000000u - m;
   const float inv = K->inv[mod];
+  constexpr float MAGIC = 12582912.0f, LIM = 4194304.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 4; ++j) {
+      float f[16], top = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        f[e] = (float)acc[i][j][e];
+        top = fmaxf(top, fabsf(f[e]));
+      }
+      if (__any(top >= LIM)) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          acc[i][j][e] -= (int)m * (int)rintf(f[e] * inv);
+          f[e] = (float)acc[i][j][e];
+        }
+      }
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         // lane (c, h) holds rows 8 g + 4 h .. + 3 of column c
         unsigned b[4];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          int x = acc[i][j][4 * g + v];
-          x -= m * (int)rintf((float)x * inv);    // the float's rounding leaves |x| < 2 m
-          x -= m * (int)rintf((float)x * inv);
-          b[v] = (unsigned)x;
-        }
+        for (int v = 0; v < 4; ++v)
+          b[v] = (unsigned)acc[i][j][4 * g + v] + __umul24(__float_as_uint(fmaf(f[4 * g + v], inv, MAGIC)), nm);
         const unsigned lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400);
         const unsigned hi = __builtin_amdgcn_perm(b[3], b[2], 0x04000c0c);
         const int col = wn * 128 + 32 * j + (lane & 31), row = wm * 128 + 32 * i + 8 * g + 4 * (lane >> 5);
         t[col * LD + row / 4] = (int)(lo | hi);
       }
+    }
   __syncthreads();
   signed char *R = G.R + mod * G.pr + (size_t)nt * CRT_T * G.ldr + (size_t)mt * CRT_T;
 #pragma unroll 4

@@ -93,8 +93,10 @@ static const CrtConst &crt_const_host() {
 }
 
 // ------------------------------------------------------------------ operands
-// element (row, k) of an operand; rows are contiguous in memory
+// element (row, k) of an operand; consecutive rows, or for KMAJOR consecutive k,
+// follow each other in memory
 struct CrtMat {
+  static constexpr bool KMAJOR = false;
   const double *x;
   long long ld;
   __device__ __forceinline__ double at(long long r, long long k) const { return x[r + ld * k]; }
@@ -102,6 +104,7 @@ struct CrtMat {
 // X(g, p) X(g, q) of column k's orbital pair (p, q), halved for p = q, zero for
 // padding columns (p < 0)
 struct CrtPairs {
+  static constexpr bool KMAJOR = false;
   const double *x;
   long long ld;
   const int *pq;
@@ -110,6 +113,25 @@ struct CrtPairs {
     if (p < 0) return 0.0;
     const double v = x[r + ld * p] * x[r + ld * q];
     return p == q ? 0.5 * v : v;
+  }
+};
+
+// rows contiguous in k
+struct CrtRows {
+  static constexpr bool KMAJOR = true;
+  const double *x;
+  long long ld;
+  __device__ __forceinline__ double at(long long r, long long k) const { return x[k + ld * r]; }
+};
+// Xa(k, a) Xb(k, b) of row a + na b
+struct CrtProducts {
+  static constexpr bool KMAJOR = true;
+  const double *xa, *xb;
+  long long ld;
+  unsigned na;
+  __device__ __forceinline__ double at(long long r, long long k) const {
+    const unsigned b = (unsigned)r / na, a = (unsigned)r - b * na;
+    return xa[k + ld * a] * xb[k + ld * b];
   }
 };
 
@@ -131,6 +153,26 @@ __global__ void __launch_bounds__(256) k_crt_sumsq(Src S, long long rows, long l
     nz |= v != 0.0;
   }
   part[blockIdx.y * rows + r] = s == 0.0 && nz ? 4.9406564584124654e-324 : s;
+}
+
+// the same for rows contiguous in k, whole rows: one wave a row
+template <class Src>
+__global__ void __launch_bounds__(256) k_crt_sumsq_rows(Src S, long long rows, long long k0, long long kk, double *part) {
+  const int lane = threadIdx.x & 63;
+  const long long r = blockIdx.x * 4LL + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (r >= rows) return;
+  double s = 0.0;
+  bool nz = false;
+#pragma unroll 4
+  for (long long k = lane; k < kk; k += 64) {
+    const double v = S.at(r, k0 + k);
+    s += v * v;
+    nz |= v != 0.0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  if (lane == 0) part[r] = s;
+  if (s == 0.0 && __ballot(nz) != 0 && lane == 0) part[r] = 4.9406564584124654e-324;
 }
 
 // scale exponents s of the rows: a norm of at most 2^CRT_BITS after scaling;
@@ -161,17 +203,33 @@ template <class Src>
 __global__ void __launch_bounds__(256) k_crt_residues(Src S, long long r0, long long rows, long long k0, long long kk,
                                                       const int *__restrict__ e, long long rpad, long long nkb,
                                                       const CrtConst *__restrict__ K, c_i4 *__restrict__ out) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  // rpad and 32 nkb are multiples of 64: the grid fits exactly
   const long long rl = blockIdx.x * 64LL + lane;             // row in the chunk
   const long long kb = blockIdx.y * 4LL + w;                 // half k block: sixteen k from 16 kb
-  if (rl >= rpad || kb >= 2 * nkb) return;
   float d[4][16];
   const bool rok = rl < rows;
   const int ex = rok ? e[r0 + rl] : 0;
+  // KMAJOR: the 64 x 64 elements through LDS, a row of 64 k at a time (rows
+  // padded by one against bank conflicts); a lane's own sixteen would touch 64
+  // lines a load
+  __shared__ double tile[Src::KMAJOR ? 64 * 65 : 1];
+  if constexpr (Src::KMAJOR) {
+    const long long k = blockIdx.y * 64LL + lane;
+#pragma unroll 4
+    for (int i = 0; i < 16; ++i) {
+      const int ri = 16 * w + i;
+      const long long r = blockIdx.x * 64LL + ri;
+      tile[ri * 65 + lane] = r < rows && k < kk ? S.at(r0 + r, k0 + k) : 0.0;
+    }
+    __syncthreads();
+  }
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const long long k = 16 * kb + i;
-    double y = rok && k < kk ? S.at(r0 + rl, k0 + k) : 0.0;
+    double y;
+    if constexpr (Src::KMAJOR) y = tile[lane * 65 + 16 * w + i];
+    else y = rok && k < kk ? S.at(r0 + rl, k0 + k) : 0.0;
     y = rint(ldexp(y, ex));
     const double y3 = rint(y * 0x1p-45);
     y = fma(-y3, 0x1p45, y);
@@ -418,8 +476,7 @@ struct CrtWork {
 static CrtWork &crt_work(Context &C) {
   if (!C.crtw) {
     C.crtw = new CrtWork();
-    C.crtw->K.upload(&crt_const_host(), 1, C.stream);
-    C.wait();
+    C.crtw->K.upload(&crt_const_host(), 1, C.stream);   // from memory that stays
   }
   return *C.crtw;
 }
@@ -440,12 +497,28 @@ bool crt_pays(long long m, long long n, long long k, double part) {
   return 28.6 * mac > 14.0 * pad + 6500.0 * (double)(m + n) * k + 5000.0 * (double)m * n + 1e11;
 }
 
+// The same for crt_products_tn.  DGEMM takes 34 fs a multiply-add on the shapes
+// of Rkab (51 to 65 TFLOP/s), and as k is short here, the number of points, the
+// ends of the tiles weigh more: 9500 fs a result element.  (H2O)n, 375 n vectors
+// of 225 n^2 pairs at 188 n points, DGEMM and int8: n = 5 442 and 446 us, n = 6
+// 807 and 727 us, n = 8 2.39 and 1.82 ms, n = 12 10.2 and 6.3 ms.  The line lies
+// 400 us higher, what a context's first call pays for the work arrays.
+bool crt_products_pay(long long m, long long n, long long k) {
+  if (m < 512 || n < 512 || k < 512) return false;
+  const double mac = (double)m * n * k, pad = (double)crt_up(m, CRT_T) * crt_up(n, CRT_T) * crt_up(k, CRT_KS);
+  return 34.0 * mac > 14.0 * pad + 6500.0 * (double)(m + n) * k + 9500.0 * (double)m * n + 5e11;
+}
+
 template <class Src>
 static void crt_exponents(Context &C, CrtWork &W, const Src &S, long long rows, long long k0, long long kk, int *e) {
-  const int slices = (int)((kk + CRT_KSUM - 1) / CRT_KSUM);
+  const int slices = Src::KMAJOR ? 1 : (int)((kk + CRT_KSUM - 1) / CRT_KSUM);
   W.part.alloc((size_t)slices * rows);
-  hipLaunchKernelGGL(k_crt_sumsq<Src>, dim3((unsigned)((rows + 255) / 256), (unsigned)slices), dim3(256), 0, C.stream,
-                     S, rows, k0, kk, W.part.p);
+  if constexpr (Src::KMAJOR)
+    hipLaunchKernelGGL(k_crt_sumsq_rows<Src>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, C.stream, S, rows, k0, kk,
+                       W.part.p);
+  else
+    hipLaunchKernelGGL(k_crt_sumsq<Src>, dim3((unsigned)((rows + 255) / 256), (unsigned)slices), dim3(256), 0, C.stream,
+                       S, rows, k0, kk, W.part.p);
   hipLaunchKernelGGL(k_crt_exps, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, C.stream, W.part.p, rows, slices,
                      e, W.bad.p);
   GI_HIP(hipGetLastError());
@@ -483,12 +556,13 @@ static bool crt_product(Context &C, const SrcA &A, const SrcB &B, long long m, l
   C.read(&bad, W.bad.p, sizeof(bad));
   if (bad) return false;
   // the smaller operand's residues stay for a chunk of k, the larger one passes
-  // in slices of about CRT_SLICE bytes, whole multiples of eight tiles, at
-  // least CRT_ROWS rows (a launch that fills the card)
-  constexpr long long CRT_SLICE = 3LL << 29, CRT_ROWS = 2048;
+  // in slices of about CRT_SLICE bytes (CRT_SLICE_R of residues of the result),
+  // whole multiples of eight tiles, at least CRT_ROWS rows (a launch that fills
+  // the card)
+  constexpr long long CRT_SLICE = 3LL << 29, CRT_SLICE_R = 4LL << 30, CRT_ROWS = 2048;
   const bool keep_a = mp <= np;
   const long long kp = std::min(kc, crt_up(k, CRT_KS));
-  long long step = CRT_SLICE / (CRT_N * kp) / (8 * CRT_T) * (8 * CRT_T);
+  long long step = std::min(CRT_SLICE / (CRT_N * kp), CRT_SLICE_R / (CRT_N * std::min(mp, np))) / (8 * CRT_T) * (8 * CRT_T);
   step = std::min(keep_a ? np : mp, std::max(step, CRT_ROWS));
   W.A.alloc((size_t)((keep_a ? mp : step) * kp / 16 * CRT_N));
   W.B.alloc((size_t)((keep_a ? step : np) * kp / 16 * CRT_N));
@@ -540,6 +614,12 @@ bool crt_gemm_nt(Context &C, long long m, long long n, long long k, double alpha
 bool crt_pairs_nt(Context &C, long long m, long long n, long long k, double alpha, const double *X, long long ldx,
                   const int *pq, const double *B, long long ldb, double beta, double *Cd, long long ldc) {
   return crt_product(C, CrtPairs{X, ldx, pq}, CrtMat{B, ldb}, m, n, k, alpha, beta, Cd, ldc, false);
+}
+
+bool crt_products_tn(Context &C, long long m, long long na, long long nb, long long k, const double *A, long long lda,
+                     const double *Xa, const double *Xb, long long ldx, double *Cd, long long ldc) {
+  if (na * nb >= (1LL << 31)) return false;
+  return crt_product(C, CrtRows{A, lda}, CrtProducts{Xa, Xb, ldx, (unsigned)na}, m, na * nb, k, 1.0, 0.0, Cd, ldc, false);
 }
 
 }  // namespace gi

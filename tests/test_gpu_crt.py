@@ -97,3 +97,21 @@ def test_non_finite_points_are_not_scaled(built):
         pass
     Z, _ = c.thc_z(X)
     assert np.isfinite(Z).all()
+
+
+@pytest.mark.parametrize("points,nvec,na,nb", [(2177, 2817, 40, 300), (900, 6001, 100, 200), (1999, 4099, 25, 425)])
+def test_rkab_products(built, points, nvec, na, nb):
+    """Rkab = Z^T (Xa o Xb) at ragged tiles, sampled against extended precision."""
+    c, b, _, _ = built
+    rng = np.random.default_rng(points)
+    X = np.asfortranarray(rng.standard_normal((points, b.nao)) * np.exp(-20.0 * rng.random((points, b.nao)) ** 2))
+    Z = np.asfortranarray(rng.standard_normal((points, nvec)))
+    C = np.asfortranarray(np.eye(b.nao)[:, rng.permutation(b.nao)])   # orbitals are columns of X, to the last bit
+    got = c.thc_rkab(X, Z, C, 1, na, C, na + 1, na + nb, 0).reshape(nvec, na, nb, order="F")
+    Y = X @ C
+    k = np.unique(np.concatenate([[0, 255, 256, nvec - 1], rng.choice(nvec, 30, replace=False)]))
+    a, q = rng.integers(0, na, 40), rng.integers(0, nb, 40)
+    a[:2], q[:2] = [0, na - 1], [0, nb - 1]
+    A, B = Z[:, k].T, (Y[:, a] * Y[:, na + q]).T
+    ref = _exact(A, B)
+    assert (np.abs(got[np.ix_(k, range(na), range(nb))][:, a, q] - ref) <= _bar(A, B, ref)).all()

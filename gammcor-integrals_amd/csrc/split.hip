@@ -33,8 +33,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int SPL_S = 4;      // slices per element
 constexpr int SPL_KC = 256;   // k per FP32 chunk; k is padded to a multiple
-constexpr int SPL_BM = 64;    // workgroup tile rows: 2 waves x 32
+constexpr int SPL_BM = 128;   // workgroup tile rows: 4 waves x 32
 constexpr int SPL_BN = 128;   // workgroup tile columns: 2 waves x 64
+constexpr int SPL_W = 8;      // waves of a workgroup
 constexpr int SPL_T = 32;     // slicing tile: 32 rows x one chunk of k
 
 // eight scaled elements (|a| < 256) into the slices of unit u
@@ -139,10 +140,15 @@ __global__ __launch_bounds__(256) void k_slice_cols(const double *__restrict__ X
 
 // C(r, c) = beta C + alpha sum_chunks 2^(ea + eb) sum_k x_r(k) y_c(k), x and y
 // the slice sums of the rows of A (mpad rows) and B (npad rows), both in the
-// fragment order of the slices, ea and eb their chunk exponents.  Workgroup: 4 waves, tile 64 x 128 (4 row
-// and 8 column blocks of 16); wave: 32 x 64 as 2 x 4 MFMA 16x16x32 blocks.
-// The 48 fragments of a 32-k step (4 + 8 blocks x 4 slices, 1 KB each) are
-// copied global -> LDS by the four waves (global_load_lds, 16 bytes per
+// fragment order of the slices, ea and eb their chunk exponents.
+// Workgroup: 8 waves, tile 128 x 128 (8 row
+// and 8 column blocks of 16); wave: 32 x 64 as 2 x 4 MFMA 16x16x32 blocks, two
+// waves per SIMD.  A step is 2560 cycles of MFMA per SIMD and 64 KB from L2;
+// four waves on 64 x 128 took 1280 and 48 KB, one wave per SIMD waiting for its
+// own copies, 1.5 us a step where the products need 0.6.  624,720 x 600 x 1200:
+// 11.5 -> 8.7 ms, 1.18 PFLOP/s.
+// The 64 fragments of a 32-k step (8 + 8 blocks x 4 slices, 1 KB each) are
+// copied global -> LDS by the eight waves (global_load_lds, 16 bytes per
 // lane, no registers), double-buffered: step s + 1 loads while step s
 // multiplies.  Lane l feeds row (column) l % 16 of a block and the eight k
 // at 8 (l / 16) of the step; it holds rows 4 (l / 16) + v, column l % 16 of
@@ -150,26 +156,19 @@ __global__ __launch_bounds__(256) void k_slice_cols(const double *__restrict__ X
 // stores are bounded by m x n.
 constexpr int SPL_NF = (SPL_BM / 16 + SPL_BN / 16) * SPL_S;   // fragments per k step
 
-__device__ static inline void stage_step(bf16x8 (*st)[64], const bf16x8 *__restrict__ A,
-                                         const bf16x8 *__restrict__ B, size_t pa, size_t pb, long long rb0,
-                                         long long cb0, long long nks, long long kk, int w, int lane) {
+// A wave copies the four slices of two blocks, from src (its first block and
+// slice, the same in every lane) for step kk on
+__device__ static inline void stage_step(bf16x8 (*st)[64], const bf16x8 *__restrict__ src, size_t plane, long long nks,
+                                         long long kk, int w, int lane) {
 #pragma unroll
-  for (int q = 0; q < SPL_NF / 4; ++q) {
-    const int f = w * (SPL_NF / 4) + q;
-    const bf16x8 *src;
-    if (f < (SPL_BM / 16) * SPL_S) {
-      const int rb = f / SPL_S, t = f % SPL_S;
-      src = A + t * pa + ((size_t)(rb0 + rb) * nks + kk) * 64 + lane;
-    } else {
-      const int g = f - (SPL_BM / 16) * SPL_S, cb = g / SPL_S, t = g % SPL_S;
-      src = B + t * pb + ((size_t)(cb0 + cb) * nks + kk) * 64 + lane;
-    }
-    __builtin_amdgcn_global_load_lds((const void *)src, (void __attribute__((address_space(3))) *)(&st[f][0]), 16, 0,
-                                     0);
+  for (int q = 0; q < 2 * SPL_S; ++q) {
+    const bf16x8 *p = src + (q % SPL_S) * plane + ((q / SPL_S) * nks + kk) * 64;
+    __builtin_amdgcn_global_load_lds((const void *)(p + lane),
+                                     (void __attribute__((address_space(3))) *)(&st[w * 2 * SPL_S + q][0]), 16, 0, 0);
   }
 }
 
-__global__ __launch_bounds__(256) void k_split_gemm(const bf16x8 *__restrict__ A, const bf16x8 *__restrict__ B,
+__global__ __launch_bounds__(64 * SPL_W) void k_split_gemm(const bf16x8 *__restrict__ A, const bf16x8 *__restrict__ B,
                                                     const int *__restrict__ ea, const int *__restrict__ eb,
                                                     long long mpad, long long npad, long long kpad, long long m,
                                                     long long n, double alpha, double beta, double *__restrict__ C,
@@ -184,10 +183,10 @@ __global__ __launch_bounds__(256) void k_split_gemm(const bf16x8 *__restrict__ A
   const long long xcd = blockIdx.x % 8, slot = blockIdx.x / 8;
   const long long rt = (slot / nct) * 8 + xcd, ct = slot % nct;
   if (rt >= nrt) return;   // whole workgroup, before any barrier
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lr = lane & 15, lg = lane >> 4;
   const long long rb0 = rt * (SPL_BM / 16), cb0 = ct * (SPL_BN / 16);
-  const int wr = (w & 1) * 2, wc = (w >> 1) * 4;   // the wave's first row / column block in the tile
+  const int wr = (w & 3) * 2, wc = (w >> 2) * 4;   // the wave's first row / column block in the tile
   const long long nks = kpad / 32;
   const size_t pa = (size_t)(mpad / 16) * nks * 64, pb = (size_t)(npad / 16) * nks * 64;
   const long long row0 = rb0 * 16 + wr * 16, col0 = cb0 * 16 + wc * 16;
@@ -198,7 +197,11 @@ __global__ __launch_bounds__(256) void k_split_gemm(const bf16x8 *__restrict__ A
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[i][j][v] = 0.0;
-  stage_step(lds[0], A, B, pa, pb, rb0, cb0, nks, 0, w, lane);
+  static_assert(SPL_NF == 2 * SPL_S * SPL_W, "two blocks a wave");
+  const bool ina = 2 * w < SPL_BM / 16;
+  const bf16x8 *src = ina ? A + (size_t)(rb0 + 2 * w) * nks * 64 : B + (size_t)(cb0 + 2 * w - SPL_BM / 16) * nks * 64;
+  const size_t plane = ina ? pa : pb;
+  stage_step(lds[0], src, plane, nks, 0, w, lane);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   for (long long kc = 0; kc < nks; kc += SPL_KC / 32) {
@@ -207,35 +210,43 @@ __global__ __launch_bounds__(256) void k_split_gemm(const bf16x8 *__restrict__ A
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) l2[i][j] = l3[i][j] = l4[i][j] = l5[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
+#pragma unroll 1
     for (int ks = 0; ks < SPL_KC / 32; ++ks) {
       const long long kk = kc + ks;
       const int cur = (int)(kk & 1);
-      if (kk + 1 < nks) stage_step(lds[cur ^ 1], A, B, pa, pb, rb0, cb0, nks, kk + 1, w, lane);
-      // fragments read slice by slice and products issued level by level
-      // over all eight blocks, so that each MFMA waits only for the slices
-      // it uses and consecutive MFMAs update different accumulators
-      bf16x8 a[2][SPL_S], b[4][SPL_S];
+      if (kk + 1 < nks) stage_step(lds[cur ^ 1], src, plane, nks, kk + 1, w, lane);
+      // the row fragments stay, a column slice is read, multiplied and
+      // dropped: all 24 fragments beside the accumulators (128 registers of
+      // levels, 64 of sums) would not fit two waves per SIMD.  Consecutive
+      // MFMAs update different accumulators.
+      bf16x8 a[2][SPL_S], b[4];
 #pragma unroll
-      for (int t = 0; t < SPL_S; ++t) {
+      for (int t = 0; t < SPL_S; ++t)
 #pragma unroll
         for (int i = 0; i < 2; ++i) a[i][t] = lds[cur][(wr + i) * SPL_S + t][lane];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b[j][t] = lds[cur][(SPL_BM / 16 + wc + j) * SPL_S + t][lane];
-      }
-#define SPL_PRODUCT(L, T, U)                                                                          \
+#define SPL_COLUMN(U)                                                                               \
+  _Pragma("unroll") for (int j = 0; j < 4; ++j) b[j] = lds[cur][(SPL_BM / 16 + wc + j) * SPL_S + U][lane];
+#define SPL_PRODUCT(L, T)                                                                             \
   _Pragma("unroll") for (int i = 0; i < 2; ++i) _Pragma("unroll") for (int j = 0; j < 4; ++j) L[i][j] = \
-      __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][T], b[j][U], L[i][j], 0, 0, 0);
-      SPL_PRODUCT(l2, 0, 0)
-      SPL_PRODUCT(l3, 0, 1)
-      SPL_PRODUCT(l3, 1, 0)
-      SPL_PRODUCT(l4, 1, 1)
-      SPL_PRODUCT(l4, 0, 2)
-      SPL_PRODUCT(l4, 2, 0)
-      SPL_PRODUCT(l5, 1, 2)
-      SPL_PRODUCT(l5, 2, 1)
-      SPL_PRODUCT(l5, 0, 3)
-      SPL_PRODUCT(l5, 3, 0)
+      __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i][T], b[j], L[i][j], 0, 0, 0);
+      SPL_COLUMN(0)
+      SPL_PRODUCT(l2, 0)
+      SPL_PRODUCT(l3, 1)
+      SPL_PRODUCT(l4, 2)
+      SPL_PRODUCT(l5, 3)
+      __builtin_amdgcn_sched_barrier(0);
+      SPL_COLUMN(1)
+      SPL_PRODUCT(l3, 0)
+      SPL_PRODUCT(l4, 1)
+      SPL_PRODUCT(l5, 2)
+      __builtin_amdgcn_sched_barrier(0);
+      SPL_COLUMN(2)
+      SPL_PRODUCT(l4, 0)
+      SPL_PRODUCT(l5, 1)
+      __builtin_amdgcn_sched_barrier(0);
+      SPL_COLUMN(3)
+      SPL_PRODUCT(l5, 0)
+#undef SPL_COLUMN
 #undef SPL_PRODUCT
       // the next step's fragments have landed and every wave is done with
       // this step's buffer before it is refilled; the scheduling barrier
@@ -320,7 +331,7 @@ void split_bf16_gemm(Context &C, rocblas_operation ta, rocblas_operation tb, lon
   const long long nwg = 8 * ((nrt + 7) / 8) * nct;
   if (nwg > 0x7fffffffLL) throw Error{63, "split product: dimension beyond the launch grid"};
   dim3 grid((unsigned)nwg);
-  hipLaunchKernelGGL(k_split_gemm, grid, dim3(256), 0, C.stream, pa, pb, ea, eb, mpad, npad, kpad, m, n, alpha, beta,
+  hipLaunchKernelGGL(k_split_gemm, grid, dim3(64 * SPL_W), 0, C.stream, pa, pb, ea, eb, mpad, npad, kpad, m, n, alpha, beta,
                      Cd, ldc);
   GI_HIP(hipGetLastError());
 }

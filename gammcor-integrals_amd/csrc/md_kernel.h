@@ -282,23 +282,28 @@ __global__ void __launch_bounds__(64) md_kernel(MdArgs A) {
   const int G = gridDim.x;
   const int w = blockIdx.x;
   const long long v0 = (G % 8 == 0) ? (long long)(w % 8) * (G / 8) + w / 8 : w;
-  const long long nct = (A.mode == LAUNCH_PRODUCT) ? (A.ncols + A.kt - 1) / A.kt : 1;
+  // tiles of a bra pair: groups of kt ket pairs, or for a diagonal its kt
+  // groups of 16-column slices, slice c in tile c % kt
+  const long long nct = (A.mode == LAUNCH_PRODUCT) ? (A.ncols + A.kt - 1) / A.kt : (A.mode == LAUNCH_DIAG ? A.kt : 1);
   const long long rs = A.trans ? A.ldo : 1;   // destination stride of a kernel row
 
   for (long long t = v0; t < A.ntiles; t += G) {
     long long ir, jc0;
-    int nk;
+    int nk, cfirst = 0, cstep = 16;
     if (A.mode == LAUNCH_PRODUCT) {
       ir = t / nct;
       jc0 = (t - ir * nct) * A.kt;
       nk = (int)((A.ncols - jc0) < A.kt ? (A.ncols - jc0) : A.kt);
     } else {
-      ir = t;
-      jc0 = t;
+      ir = t / nct;
+      jc0 = ir;
       nk = 1;
+      cfirst = 16 * (int)(t - ir * nct);
+      cstep = 16 * (int)nct;
     }
     const QRec RB = A.rrec[ir];
     const int nr = RB.nrow;
+    if (A.mode == LAUNCH_DIAG && cfirst >= nr) continue;   // the pair has fewer slices
     const int ldb = RB.n0 * RB.n1;
     int fr[RT];
 #pragma unroll
@@ -377,7 +382,7 @@ __global__ void __launch_bounds__(64) md_kernel(MdArgs A) {
         const bool single = (CD.nprim == 1);
         if (single) rtable<E + F>(s_R[0], s_R[1], PB, first_prim(CD), A.kappa, A.boys, lane, s_rrec);
 
-        for (int c0 = 0; c0 < nc; c0 += 16) {
+        for (int c0 = cfirst; c0 < nc; c0 += cstep) {
           const int cc = c0 + i16;
           const int ncs = (nc - c0) < 16 ? (nc - c0) : 16;
           if (ncs <= MD_NCV && A.mode != LAUNCH_DIAG) {

@@ -21,8 +21,8 @@
 // down to 1.6 GHz), where DGEMM takes 28.6 fs at 70 TFLOP/s.  Norms, conversion
 // and reconstruction move 31 bytes per operand element and up to 38 per result
 // element at memory speed and take back a part (crt_pays).  (H2O)16, 1200 AOs,
-// 7809 vectors of 316,063 pairs: vectors' product 287 -> 170 ms, SubtractR 84 ->
-// 64 ms; XR of 1536 points 115 -> 46 ms.
+// 7809 vectors of 316,063 pairs: vectors' product 287 -> 165 ms, SubtractR 84 ->
+// 62 ms; XR of 1536 points 115 -> 45 ms.
 //
 // Layout.  Residues of an operand: [modulus][32-row block][32-k block] fragments
 // of 1 KB, lane l of v_mfma_i32_32x32x32_i8 holding row l % 32 and the sixteen k

@@ -201,7 +201,7 @@ __global__ void __launch_bounds__(64) k_thc_pivot_max(const double *__restrict__
 // With the whole of D scanned by every workgroup, a tree of ten barriers and
 // the elements fetched after it a step took 11.8 us at 9600 candidates; 4.7 us
 // here, and about 2.5 us between two launches.  Pruning 9600 points (6000
-// pivots, 600 AOs): 92 -> 57 ms.
+// pivots, 600 AOs): 92 -> 57 ms, 52 with the Schur complement's lower part only.
 constexpr int PIV_PANEL = 128;   // Schur form: vectors kept outside Shat
 // Schur form: columns of a block column of Shat.  A DGEMM of the whole square
 // updates every element twice (43 of 378 us, 16.3 of 54 ms, when 9600 points are

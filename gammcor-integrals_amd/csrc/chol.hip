@@ -1382,8 +1382,9 @@ void chol_build(Context &C, double tau, double kappa, long long max_block_dim, l
     const size_t slab = (size_t)msd * nvec;
     // 64 doubles behind the last column: the MO transform reads whole 64-vector tiles
     S.rkpq.alloc((size_t)nvec * msd * nsub + 64);
-    // subsets per group: keep the Vabrs staging under ~16 GiB
-    long long per_group = std::max<long long>(1, (long long)((16.0 * (1ull << 30)) / (8.0 * (double)std::max<size_t>(slab, 1))));
+    // subsets per group: keep the Vabrs staging under vec_stage_mb
+    long long per_group =
+        std::max<long long>(1, (long long)(C.vec_stage_mb * 1048576.0 / (8.0 * (double)std::max<size_t>(slab, 1))));
     per_group = std::min(per_group, nsub);
     DBuf<double> &dW = chol_work(C).Wv;
     dW.alloc(slab * per_group);

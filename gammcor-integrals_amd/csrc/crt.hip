@@ -274,7 +274,8 @@ struct CrtGemm {
   int nkb;                  // 32-k blocks (even)
   int nmt, nnt;             // tiles of rows and columns
   long long ldr;            // rows of a column of R
-  int tri;                  // rows of A end with their diagonal: row tile t needs k < 256 (t + 1)
+  int tri;                  // rows of A end with their diagonal: row tile t of all needs k < 256 (t + 1)
+  int mt0;                  // row tiles of A before the first one held here
 };
 
 // Residue products modulo crt_mod(blockIdx.y): 256 x 256 tiles, four waves of
@@ -308,7 +309,8 @@ __global__ void __launch_bounds__(256, 1) k_crt_gemm(CrtGemm G, const CrtConst *
   }
   const int wm = w & 1, wn = w >> 1;
   int nks = G.nkb / 2;
-  if (G.tri && (mt + 1) * (CRT_T / CRT_KS) < nks) nks = (mt + 1) * (CRT_T / CRT_KS);
+  const int diag = (G.mt0 + mt + 1) * (CRT_T / CRT_KS);
+  if (G.tri && diag < nks) nks = diag;
   // this wave's copies: 32-row blocks 4 w .. 4 w + 3 of the tile's sixteen (A, then B)
   const c_i4 *src[4];
 #pragma unroll
@@ -556,13 +558,14 @@ static bool crt_product(Context &C, const SrcA &A, const SrcB &B, long long m, l
   C.read(&bad, W.bad.p, sizeof(bad));
   if (bad) return false;
   // the smaller operand's residues stay for a chunk of k, the larger one passes
-  // in slices of about CRT_SLICE bytes (CRT_SLICE_R of residues of the result),
-  // whole multiples of eight tiles, at least CRT_ROWS rows (a launch that fills
-  // the card)
-  constexpr long long CRT_SLICE = 3LL << 29, CRT_SLICE_R = 4LL << 30, CRT_ROWS = 2048;
+  // in slices of about a sixth of the work arrays' bytes (four ninths for the
+  // residues of the result), whole multiples of eight tiles, at least CRT_ROWS
+  // rows (a launch that fills the card)
+  constexpr long long CRT_ROWS = 2048;
+  const long long work = C.int8_work_mb << 20, slice = work / 6, slice_r = work / 9 * 4;
   const bool keep_a = mp <= np;
   const long long kp = std::min(kc, crt_up(k, CRT_KS));
-  long long step = std::min(CRT_SLICE / (CRT_N * kp), CRT_SLICE_R / (CRT_N * std::min(mp, np))) / (8 * CRT_T) * (8 * CRT_T);
+  long long step = std::min(slice / (CRT_N * kp), slice_r / (CRT_N * std::min(mp, np))) / (8 * CRT_T) * (8 * CRT_T);
   step = std::min(keep_a ? np : mp, std::max(step, CRT_ROWS));
   W.A.alloc((size_t)((keep_a ? mp : step) * kp / 16 * CRT_N));
   W.B.alloc((size_t)((keep_a ? step : np) * kp / 16 * CRT_N));
@@ -591,6 +594,7 @@ static bool crt_product(Context &C, const SrcA &A, const SrcB &B, long long m, l
       G.nnt = (int)(bn / CRT_T);
       G.ldr = am;
       G.tri = tri ? 1 : 0;
+      G.mt0 = keep_a ? 0 : (int)(s0 / CRT_T);   // slices are whole tiles
       const long long big = std::max(G.nmt, G.nnt), small = std::min(G.nmt, G.nnt);
       hipLaunchKernelGGL(k_crt_gemm, dim3((unsigned)(8 * ((big + 7) / 8) * small), CRT_N), dim3(256), 0, C.stream, G,
                          W.K.p);

@@ -177,6 +177,9 @@ struct Context {
   // THC grid pruning: the explicit Schur-complement form is used once the
   // candidates' ncand^2 doubles fit this many MiB (0: never)
   long long thc_schur_mb = 24576;
+  // work arrays of the int8 products (crt.hip), and the staging of Vabrs for
+  // the full-dimension vectors (at least one subset), in MiB
+  long long int8_work_mb = 9216, vec_stage_mb = 16384;
   // THC least-squares Z: Cholesky of the metric first (LU when a pivot is not
   // positive); 0 always solves by LU
   int thc_cholesky = 1;

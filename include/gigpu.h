@@ -131,6 +131,11 @@ int gi_eri_pair_block(gi_context *ctx, int64_t nrow_pairs, const int64_t *row_pa
  *   "thc_schur_mb"   gi_thc_grid_pivots keeps the Schur complement of S over
  *                    the candidates explicitly once it fits this many MiB
  *                    (24576; 0: columns built on the fly throughout)
+ *   "int8_work_mb"   work arrays of the large products on the int8 matrix
+ *                    cores, MiB (9216): operands pass in slices that fit
+ *   "vec_stage_mb"   staging of Vabrs for the full-dimension vectors, MiB
+ *                    (16384): subsets are formed in groups that fit, at least
+ *                    one subset each
  *   "thc_cholesky"   gi_thc_z factors S by Cholesky first, LU when a pivot
  *                    is not positive (1); 0: LU always
  * Unknown names fail.  Results do not depend on these settings beyond

@@ -1,0 +1,64 @@
+"""Products on the int8 matrix cores (crt.hip) whose larger operand passes in
+several slices: the vectors Inv_L V(P, pq) of a decomposition with more vectors
+than columns in a subset, where the slices are rows of the triangular Inv_L.
+
+The bar is the scheme's own, as in test_gpu_crt.py: half a unit an element at
+row norms of 2^57..2^58 units, sqrt(k) 2^-57 |a| |b|, plus one rounding of the
+result and the reference's own."""
+import numpy as np
+import pytest
+import torch
+
+from gigpu import lib, systems
+
+pytestmark = pytest.mark.gpu
+
+
+class _Device:
+    def __init__(self, pointer, shape):
+        self.__cuda_array_interface__ = {"shape": shape, "typestr": "<f8", "data": (pointer, False), "strides": None,
+                                         "version": 2}
+
+
+def _check_vectors(c, b):
+    """Sampled elements of Rkpq, rows from every tile column of 256, against extended precision."""
+    m, X = c.chol_meta(), c.chol_inv_l()
+    nv, msd = m["nvecs"], m["max_subset_dim"]
+    R = torch.as_tensor(_Device(c.chol_rkpq_device_ptr(), (m["nsubsets"], msd, nv)), device="cuda")
+    sp, loc = m["shell_pairs"], m["shell_pair_loc"]
+    piv = [tuple(sp[i - 1] - 1) for i in m["pivot_shell_pairs"]]
+    sel, off, k = [], 0, 0
+    for (p, q), n in zip(piv, m["pivot_shell_pair_dim"]):
+        sel += [off + m["pivot_orb_pairs"][k + j] - 1 for j in range(n)]
+        k += n
+        off += b.shell_nang(p) * b.shell_nang(q)
+    rng = np.random.default_rng(7)
+    pick = [s for s in [0, 1, len(sp) - 2, len(sp) - 1] + list(rng.choice(len(sp), 8, replace=False))
+            if sp[s][0] != sp[s][1]]
+    V = c.eri_pair_block([tuple(sp[s] - 1) for s in pick], piv)[:, sel]
+    rows = np.unique(np.concatenate([np.arange(0, nv, 256), np.arange(255, nv, 256), [nv - 1]]))
+    at = torch.from_numpy(rows).cuda()
+    got = np.concatenate([R[loc[s][2] - 1, loc[s][1] - 1:loc[s][1] - 1 + m["shell_pair_dim"][s]][:, at].cpu().numpy()
+                          for s in pick]).T
+    A = X[rows]
+    ref = np.asarray(A, np.longdouble) @ np.asarray(V, np.longdouble).T
+    bar = (np.sqrt(nv) * 2.0 ** -57 * np.linalg.norm(A, axis=1)[:, None] * np.linalg.norm(V, axis=1)[None, :]
+           + 2.0 ** -52 * np.abs(ref) + np.sqrt(nv) * 2.0 ** -63 * (np.abs(A) @ np.abs(V).T)).astype(float)
+    err = np.abs(got - ref).astype(float)
+    assert (err <= bar).all(), (float((err / bar).max()), rows[(err > bar).any(axis=1)][:8])
+
+
+def test_triangular_rows_in_slices():
+    b = systems.water_system(6, 7.2, "large", seed=41)
+    c = lib.Context(0)
+    try:
+        c.set_basis(b)
+        c.set_option("vec_stage_mb", 1)   # a product for every subset of at most 4003 columns
+        c.set_option("int8_work_mb", 1)   # slices of 2048 rows, the smallest
+        c.chol_build(tau=1e-10)
+        d = c.chol_dims()
+        # more rows than columns, in three slices; the int8 route is the faster one from 4800 x 3600 on
+        assert d["nvecs"] > 4800 and d["nvecs"] % 256 != 0 and 3600 < d["max_subset_dim"] < d["nvecs"]
+        _check_vectors(c, b)
+    finally:
+        c.close()

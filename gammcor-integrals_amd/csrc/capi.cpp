@@ -35,7 +35,7 @@ using gi::Error;
 static gi::Context &ctx_of(gi_context *c) {
   if (!c || !c->c) throw Error{7, "null gi_context"};
   GI_HIP(hipSetDevice(c->c->device));
-  gi::g_alloc_stream = c->c->stream;
+  c->c->enter();
   return *c->c;
 }
 
@@ -223,7 +223,10 @@ int gi_set_option(gi_context *cp, const char *name, int64_t value) {
     else if (n == "micro_persist_max") C.micro_persist_max = std::max<int64_t>(0, value);
     else if (n == "grad_screen") C.grad_screen = std::min<int64_t>(30, std::max<int64_t>(0, value));
     else if (n == "thc_schur_mb") C.thc_schur_mb = std::max<int64_t>(0, value);
-    else if (n == "int8_work_mb") C.int8_work_mb = std::min<int64_t>(1 << 20, std::max<int64_t>(1, value));
+    else if (n == "int8_work_mb") {
+      C.int8_work_mb = std::min<int64_t>(1 << 20, std::max<int64_t>(0, value));
+      gi::release_crt_work(C);   // the next product allocates what it may now have
+    }
     else if (n == "vec_stage_mb") C.vec_stage_mb = std::min<int64_t>(1 << 20, std::max<int64_t>(1, value));
     else if (n == "thc_cholesky") C.thc_cholesky = value != 0;
     else if (n == "eri_lane_emax") C.eri_lane_emax = std::max<int64_t>(0, value);

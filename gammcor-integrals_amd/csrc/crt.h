@@ -11,7 +11,8 @@ bool crt_pays(long long m, long long n, long long k, double part = 1.0);
 // C (m x n, ldc) = beta C + alpha A B^T, A (m x k, lda) and B (n x k, ldb)
 // column-major; tri: A is lower triangular (its upper part holds zeros).
 // false, with C untouched, when an operand has rows that cannot be scaled (NaN,
-// infinities, norms outside 1e-125..1e150): the caller's DGEMM then.
+// infinities, norms outside 1e-125..1e150), or when the work arrays cannot be had
+// (int8_work_mb 0, a failed allocation): the caller's DGEMM then.
 bool crt_gemm_nt(Context &C, long long m, long long n, long long k, double alpha, const double *A, long long lda,
                  const double *B, long long ldb, double beta, double *Cd, long long ldc, bool tri);
 

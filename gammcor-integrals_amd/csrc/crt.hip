@@ -274,8 +274,8 @@ struct CrtGemm {
   int nkb;                  // 32-k blocks (even)
   int nmt, nnt;             // tiles of rows and columns
   long long ldr;            // rows of a column of R
-  int tri;                  // rows of A end with their diagonal: row tile t of all needs k < 256 (t + 1)
-  int mt0;                  // row tiles of A before the first one held here
+  int tri;                  // rows of A end with their diagonal: row tile t of the chunk needs k < 256 (t + 1)
+  int mt0;                  // the chunk's row tiles before the first one held here
 };
 
 // Residue products modulo crt_mod(blockIdx.y): 256 x 256 tiles, four waves of
@@ -467,9 +467,9 @@ __global__ void __launch_bounds__(256) k_crt_result(const signed char *__restric
 // ------------------------------------------------------------------ driver
 static long long crt_up(long long x, long long q) { return (x + q - 1) / q * q; }
 
-// Work arrays, kept in the context and grown only
+// Work arrays, kept in the context and grown only, about int8_work_mb of them
 struct CrtWork {
-  DBuf<c_i4> A, B;
+  DBuf<c_i4> keep, pass;   // residues of the operand that stays and of a slice of the other
   DBuf<signed char> R;
   DBuf<double> part;
   DBuf<int> ea, eb, bad;
@@ -512,9 +512,13 @@ bool crt_products_pay(long long m, long long n, long long k) {
 }
 
 template <class Src>
+static int crt_slices(long long kk) {   // partial sums of a row's squares
+  return Src::KMAJOR ? 1 : (int)((kk + CRT_KSUM - 1) / CRT_KSUM);
+}
+
+template <class Src>
 static void crt_exponents(Context &C, CrtWork &W, const Src &S, long long rows, long long k0, long long kk, int *e) {
-  const int slices = Src::KMAJOR ? 1 : (int)((kk + CRT_KSUM - 1) / CRT_KSUM);
-  W.part.alloc((size_t)slices * rows);
+  const int slices = crt_slices<Src>(kk);
   if constexpr (Src::KMAJOR)
     hipLaunchKernelGGL(k_crt_sumsq_rows<Src>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, C.stream, S, rows, k0, kk,
                        W.part.p);
@@ -535,17 +539,54 @@ static void crt_residues(Context &C, CrtWork &W, const Src &S, long long r0, lon
   GI_HIP(hipGetLastError());
 }
 
-// false (and C untouched) when a row cannot be scaled
+// false (and C untouched) when a row cannot be scaled, the work arrays cannot
+// be had or the option int8_work_mb is 0
 template <class SrcA, class SrcB>
 static bool crt_product(Context &C, const SrcA &A, const SrcB &B, long long m, long long n, long long k, double alpha,
                         double beta, double *Cd, long long ldc, bool tri) {
-  CrtWork &W = crt_work(C);
-  // k in chunks; the scale exponents of all chunks first
-  const long long nkc = (k + CRT_KMAX - 1) / CRT_KMAX, kc = crt_up((k + nkc - 1) / nkc, CRT_KS);
+  if (C.int8_work_mb <= 0) return false;
+  struct Busy {   // the arrays are in use: not to be given back to an allocation that fails
+    Context &C;
+    explicit Busy(Context &c) : C(c) { ++C.work_busy; }
+    ~Busy() { --C.work_busy; }
+  } busy(C);
+  // The smaller operand's residues stay for a chunk of k, the larger one passes
+  // in slices, whole multiples of eight tiles, at least CRT_ROWS rows (a launch
+  // that fills the card).  Of the work arrays' bytes a third is for the operand
+  // that stays (what is left of k goes to further chunks, each of which adds a
+  // pass over the result), a sixth for the slice, four ninths for the residues
+  // of the result.
+  constexpr long long CRT_ROWS = 2048, CRT_KMIN = 2048;
+  constexpr long long CRT_NMAX = 65535LL * 4 / CRT_ROWS * CRT_ROWS;   // columns of a k_crt_result launch
   const long long mp = crt_up(m, CRT_T), np = crt_up(n, CRT_T);
-  W.ea.alloc((size_t)(nkc * mp));
-  W.eb.alloc((size_t)(nkc * np));
-  W.bad.alloc(1);
+  const bool keep_a = mp <= np;
+  const long long small = std::min(mp, np), large = std::max(mp, np), work = C.int8_work_mb << 20;
+  const long long kmax = std::min(CRT_KMAX, std::max(CRT_KMIN, work / 3 / (CRT_N * small) / CRT_T * CRT_T));
+  const long long nkc = (k + kmax - 1) / kmax;
+  // chunks of a triangular A begin with a row tile: the rows before it end
+  // before the chunk, those from it on end at the tiles' diagonal again
+  const long long kc = crt_up((k + nkc - 1) / nkc, tri && nkc > 1 ? CRT_T : CRT_KS);
+  const long long kp = std::min(kc, crt_up(k, CRT_KS));
+  long long step = std::min(work / 6 / (CRT_N * kp), work / 9 * 4 / (CRT_N * small)) / CRT_ROWS * CRT_ROWS;
+  step = std::min({large, std::max(step, CRT_ROWS), CRT_NMAX});
+  if (!keep_a && np > CRT_NMAX) return false;
+  CrtWork *Wp;
+  try {
+    Wp = &crt_work(C);
+    Wp->ea.alloc((size_t)(nkc * mp));
+    Wp->eb.alloc((size_t)(nkc * np));
+    Wp->bad.alloc(1);
+    Wp->part.alloc((size_t)std::max(crt_slices<SrcA>(kc) * m, crt_slices<SrcB>(kc) * n));
+    Wp->keep.alloc((size_t)(small * kp / 16 * CRT_N));
+    Wp->pass.alloc((size_t)(step * kp / 16 * CRT_N));
+    Wp->R.alloc((size_t)(small * step * CRT_N));
+  } catch (const Error &) {
+    (void)hipGetLastError();
+    release_crt_work(C);
+    return false;
+  }
+  CrtWork &W = *Wp;
+  // the scale exponents of all chunks first
   const int zero = 0;
   C.h2d(W.bad.p, &zero, sizeof(zero));
   for (long long c = 0; c < nkc; ++c) {
@@ -557,52 +598,42 @@ static bool crt_product(Context &C, const SrcA &A, const SrcB &B, long long m, l
   int bad = 0;
   C.read(&bad, W.bad.p, sizeof(bad));
   if (bad) return false;
-  // the smaller operand's residues stay for a chunk of k, the larger one passes
-  // in slices of about a sixth of the work arrays' bytes (four ninths for the
-  // residues of the result), whole multiples of eight tiles, at least CRT_ROWS
-  // rows (a launch that fills the card)
-  constexpr long long CRT_ROWS = 2048;
-  const long long work = C.int8_work_mb << 20, slice = work / 6, slice_r = work / 9 * 4;
-  const bool keep_a = mp <= np;
-  const long long kp = std::min(kc, crt_up(k, CRT_KS));
-  long long step = std::min(slice / (CRT_N * kp), slice_r / (CRT_N * std::min(mp, np))) / (8 * CRT_T) * (8 * CRT_T);
-  step = std::min(keep_a ? np : mp, std::max(step, CRT_ROWS));
-  W.A.alloc((size_t)((keep_a ? mp : step) * kp / 16 * CRT_N));
-  W.B.alloc((size_t)((keep_a ? step : np) * kp / 16 * CRT_N));
-  W.R.alloc((size_t)((keep_a ? mp : step) * (keep_a ? step : np) * CRT_N));
+  c_i4 *const bufa = keep_a ? W.keep.p : W.pass.p, *const bufb = keep_a ? W.pass.p : W.keep.p;
   for (long long c = 0; c < nkc; ++c) {
     const long long k0 = c * kc, kk = std::min(kc, k - k0);
     if (kk <= 0) break;
     const int *ea = W.ea.p + c * mp, *eb = W.eb.p + c * np;
     const long long nkb = crt_up(kk, CRT_KS) / 32;
-    if (keep_a) crt_residues(C, W, A, 0, m, mp, k0, kk, ea, W.A.p);
-    else crt_residues(C, W, B, 0, n, np, k0, kk, eb, W.B.p);
-    for (long long s0 = 0; s0 < (keep_a ? n : m); s0 += step) {
-      const long long rows = std::min(step, (keep_a ? n : m) - s0), rp = crt_up(rows, CRT_T);
-      if (keep_a) crt_residues(C, W, B, s0, rows, rp, k0, kk, eb, W.B.p);
-      else crt_residues(C, W, A, s0, rows, rp, k0, kk, ea, W.A.p);
+    const long long m0 = tri ? k0 : 0;   // first row with elements in the chunk
+    if (m0 >= m) break;
+    if (keep_a) crt_residues(C, W, A, m0, m - m0, crt_up(m - m0, CRT_T), k0, kk, ea, bufa);
+    else crt_residues(C, W, B, 0, n, np, k0, kk, eb, bufb);
+    const long long end = keep_a ? n : m;
+    for (long long s0 = keep_a ? 0 : m0; s0 < end; s0 += step) {
+      const long long a0 = keep_a ? m0 : s0, am = keep_a ? m - m0 : std::min(step, end - s0);
+      const long long b0 = keep_a ? s0 : 0, bn = keep_a ? std::min(step, end - s0) : n;
+      const long long amp = crt_up(am, CRT_T), bnp = crt_up(bn, CRT_T);
+      if (keep_a) crt_residues(C, W, B, b0, bn, bnp, k0, kk, eb, bufb);
+      else crt_residues(C, W, A, a0, am, amp, k0, kk, ea, bufa);
       CrtGemm G{};
-      G.A = W.A.p;
-      G.B = W.B.p;
+      G.A = bufa;
+      G.B = bufb;
       G.R = W.R.p;
-      const long long am = keep_a ? mp : rp, bn = keep_a ? rp : np;
-      G.pa = (size_t)am / 32 * nkb * 64;
-      G.pb = (size_t)bn / 32 * nkb * 64;
-      G.pr = (size_t)am * bn;
+      G.pa = (size_t)amp / 32 * nkb * 64;
+      G.pb = (size_t)bnp / 32 * nkb * 64;
+      G.pr = (size_t)amp * bnp;
       G.nkb = (int)nkb;
-      G.nmt = (int)(am / CRT_T);
-      G.nnt = (int)(bn / CRT_T);
-      G.ldr = am;
+      G.nmt = (int)(amp / CRT_T);
+      G.nnt = (int)(bnp / CRT_T);
+      G.ldr = amp;
       G.tri = tri ? 1 : 0;
-      G.mt0 = keep_a ? 0 : (int)(s0 / CRT_T);   // slices are whole tiles
-      const long long big = std::max(G.nmt, G.nnt), small = std::min(G.nmt, G.nnt);
-      hipLaunchKernelGGL(k_crt_gemm, dim3((unsigned)(8 * ((big + 7) / 8) * small), CRT_N), dim3(256), 0, C.stream, G,
+      G.mt0 = (int)((a0 - m0) / CRT_T);   // slices are whole tiles
+      const long long big = std::max(G.nmt, G.nnt), less = std::min(G.nmt, G.nnt);
+      hipLaunchKernelGGL(k_crt_gemm, dim3((unsigned)(8 * ((big + 7) / 8) * less), CRT_N), dim3(256), 0, C.stream, G,
                          W.K.p);
-      const long long cm = keep_a ? m : rows, cn = keep_a ? rows : n;
-      double *dst = Cd + (keep_a ? ldc * s0 : s0);
-      hipLaunchKernelGGL(k_crt_result, dim3((unsigned)((cm + 255) / 256), (unsigned)((cn + 3) / 4)), dim3(256), 0,
-                         C.stream, W.R.p, G.pr, G.ldr, cm, cn, ea + (keep_a ? 0 : s0), eb + (keep_a ? s0 : 0), alpha,
-                         c == 0 ? beta : 1.0, dst, ldc, crt_const_host());
+      hipLaunchKernelGGL(k_crt_result, dim3((unsigned)((am + 255) / 256), (unsigned)((bn + 3) / 4)), dim3(256), 0,
+                         C.stream, W.R.p, G.pr, G.ldr, am, bn, ea + a0, eb + b0, alpha, c == 0 ? beta : 1.0,
+                         Cd + a0 + ldc * b0, ldc, crt_const_host());
       GI_HIP(hipGetLastError());
     }
   }
@@ -611,7 +642,6 @@ static bool crt_product(Context &C, const SrcA &A, const SrcB &B, long long m, l
 
 bool crt_gemm_nt(Context &C, long long m, long long n, long long k, double alpha, const double *A, long long lda,
                  const double *B, long long ldb, double beta, double *Cd, long long ldc, bool tri) {
-  if (tri && k > CRT_KMAX) return false;
   return crt_product(C, CrtMat{A, lda}, CrtMat{B, ldb}, m, n, k, alpha, beta, Cd, ldc, tri);
 }
 

@@ -7,6 +7,7 @@ namespace gi {
 
 static thread_local std::string g_last_error;
 thread_local hipStream_t g_alloc_stream = nullptr;
+static thread_local Context *g_ctx = nullptr;   // set with g_alloc_stream
 void set_error(const std::string &m) { g_last_error = m; }
 const char *last_error() { return g_last_error.c_str(); }
 
@@ -16,7 +17,7 @@ Context::Context(int dev) : device(dev) {
   if (dev < 0 || dev >= n) throw Error{1, "invalid HIP device index " + std::to_string(dev)};
   GI_HIP(hipSetDevice(dev));
   GI_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  g_alloc_stream = stream;
+  enter();
   // keep freed stream-ordered memory in the device pool (reused by the next
   // build instead of going back to the driver at every synchronization)
   hipMemPool_t pool = nullptr;
@@ -29,7 +30,24 @@ Context::Context(int dev) : device(dev) {
   upload_constants(*this);
 }
 
+void Context::enter() {
+  g_alloc_stream = stream;
+  g_ctx = this;
+}
+
+bool give_back_work() {
+  Context *C = g_ctx;
+  if (!C || C->work_busy > 0 || !C->crtw) return false;
+  release_crt_work(*C);
+  // the frees are stream-ordered, and the pool keeps what they return
+  (void)hipStreamSynchronize(C->stream);
+  hipMemPool_t pool = nullptr;
+  if (hipDeviceGetDefaultMemPool(&pool, C->device) == hipSuccess && pool) (void)hipMemPoolTrimTo(pool, 0);
+  return true;
+}
+
 Context::~Context() {
+  if (g_ctx == this) g_ctx = nullptr;
   (void)hipSetDevice(device);
   if (stream) (void)hipStreamSynchronize(stream);
   if (blas) rocblas_destroy_handle(blas);

@@ -20,6 +20,19 @@ namespace gi {
 // host threads never synchronize each other through allocation.
 extern thread_local hipStream_t g_alloc_stream;
 
+// An allocation has failed: frees the device arrays that the calling thread's
+// context keeps for speed only and that no call under way uses.  false: none.
+bool give_back_work();
+
+inline hipError_t device_malloc(void **p, size_t bytes, hipStream_t s) {
+  hipError_t e = hipMallocAsync(p, bytes, s);
+  if (e == hipErrorOutOfMemory && give_back_work()) {
+    (void)hipGetLastError();
+    e = hipMallocAsync(p, bytes, s);
+  }
+  return e;
+}
+
 // owning device buffer
 template <class T>
 struct DBuf {
@@ -40,7 +53,7 @@ struct DBuf {
     release();
     if (count == 0) count = 1;
     st = g_alloc_stream;
-    GI_HIP(hipMallocAsync((void **)&p, count * sizeof(T), st));
+    GI_HIP(device_malloc((void **)&p, count * sizeof(T), st));
     n = count;
   }
   void upload(const T *src, size_t count, hipStream_t s) {
@@ -53,7 +66,7 @@ struct DBuf {
     if (count <= n && p) return;
     size_t nn = std::max(count, n + n / 2);
     T *q = nullptr;
-    GI_HIP(hipMallocAsync((void **)&q, nn * sizeof(T), s));
+    GI_HIP(device_malloc((void **)&q, nn * sizeof(T), s));
     if (p && n) GI_HIP(hipMemcpyAsync(q, p, n * sizeof(T), hipMemcpyDeviceToDevice, s));
     release();
     p = q;
@@ -177,9 +190,10 @@ struct Context {
   // THC grid pruning: the explicit Schur-complement form is used once the
   // candidates' ncand^2 doubles fit this many MiB (0: never)
   long long thc_schur_mb = 24576;
-  // work arrays of the int8 products (crt.hip), and the staging of Vabrs for
-  // the full-dimension vectors (at least one subset), in MiB
+  // work arrays of the int8 products (crt.hip; 0: DGEMM instead), and the
+  // staging of Vabrs for the full-dimension vectors (at least one subset), in MiB
   long long int8_work_mb = 9216, vec_stage_mb = 16384;
+  int work_busy = 0;   // calls under way that use arrays give_back_work could free
   // THC least-squares Z: Cholesky of the metric first (LU when a pivot is not
   // positive); 0 always solves by LU
   int thc_cholesky = 1;
@@ -213,6 +227,7 @@ struct Context {
 
   Context(int dev);
   ~Context();
+  void enter();   // the calling thread works for this context from here on
 };
 
 // ---------------------------------------------------------------- ERI driver

@@ -132,7 +132,10 @@ int gi_eri_pair_block(gi_context *ctx, int64_t nrow_pairs, const int64_t *row_pa
  *                    the candidates explicitly once it fits this many MiB
  *                    (24576; 0: columns built on the fly throughout)
  *   "int8_work_mb"   work arrays of the large products on the int8 matrix
- *                    cores, MiB (9216): operands pass in slices that fit
+ *                    cores, about this many MiB (9216): operands pass in
+ *                    slices and chunks that fit.  0: FP64 matrix products
+ *                    throughout, as also when the arrays cannot be allocated.
+ *                    Setting it frees what the context holds of them
  *   "vec_stage_mb"   staging of Vabrs for the full-dimension vectors, MiB
  *                    (16384): subsets are formed in groups that fit, at least
  *                    one subset each

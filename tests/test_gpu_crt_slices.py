@@ -1,10 +1,13 @@
-"""Products on the int8 matrix cores (crt.hip) whose larger operand passes in
-several slices: the vectors Inv_L V(P, pq) of a decomposition with more vectors
-than columns in a subset, where the slices are rows of the triangular Inv_L.
+"""Products on the int8 matrix cores (crt.hip) in several slices of the larger
+operand and chunks of k: the vectors Inv_L V(P, pq) with slices of columns, or,
+for a decomposition with more vectors than columns in a subset, slices of rows
+of the triangular Inv_L; and what the context holds of their work arrays.
 
 The bar is the scheme's own, as in test_gpu_crt.py: half a unit an element at
 row norms of 2^57..2^58 units, sqrt(k) 2^-57 |a| |b|, plus one rounding of the
 result and the reference's own."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -60,5 +63,61 @@ def test_triangular_rows_in_slices():
         # more rows than columns, in three slices; the int8 route is the faster one from 4800 x 3600 on
         assert d["nvecs"] > 4800 and d["nvecs"] % 256 != 0 and 3600 < d["max_subset_dim"] < d["nvecs"]
         _check_vectors(c, b)
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("stage_mb,work_mb", [
+    (1, 1140),      # subset by subset, all of k at once: three slices of rows
+    (16384, 1140),  # all subsets at once, all of k at once: slices of 2048 columns
+    (16384, 1),     # and three chunks of k, the smallest
+])
+def test_slices_and_chunks(stage_mb, work_mb):
+    b = systems.water_system(6, 7.2, "large", seed=41)
+    c = lib.Context(0)
+    try:
+        c.set_basis(b)
+        c.set_option("int8_work_mb", 0)   # DGEMM
+        c.chol_build(tau=1e-10)
+        ref = c.chol_meta()
+        c.set_option("vec_stage_mb", stage_mb)
+        c.set_option("int8_work_mb", work_mb)
+        c.chol_build(tau=1e-10)
+        m = c.chol_meta()
+        # SubtractR goes the same ways (more rows than columns, added to M): the same pivots
+        assert m["nvecs"] == ref["nvecs"] > 4800
+        assert (m["pivot_order"] == ref["pivot_order"]).all()
+        _check_vectors(c, b)
+    finally:
+        c.close()
+
+
+def _pool_bytes():
+    """Bytes in use of the device's stream-ordered memory pool."""
+    hip = C.CDLL("libamdhip64.so")
+    pool, used = C.c_void_p(), C.c_uint64()
+    assert hip.hipDeviceGetDefaultMemPool(C.byref(pool), 0) == 0
+    assert hip.hipMemPoolGetAttribute(pool, 7, C.byref(used)) == 0   # hipMemPoolAttrUsedMemCurrent
+    return used.value
+
+
+def test_work_arrays_are_given_back():
+    """The int8 products' arrays go when the option is set, and with 0 a build
+    allocates none of them."""
+    b = systems.water_system(6, 7.2, "large", seed=41)
+    c = lib.Context(0)
+    try:
+        c.set_basis(b)
+        c.chol_build(tau=1e-5)
+        torch.cuda.synchronize()
+        held = _pool_bytes()
+        c.set_option("int8_work_mb", 0)
+        torch.cuda.synchronize()
+        freed = _pool_bytes()
+        # Inv_L's residues alone: 15 bytes an element of 2304 x 2304 at least
+        assert c.chol_dims()["nvecs"] > 2048 and held - freed >= 15 * 2304 * 2304
+        c.chol_build(tau=1e-5)
+        torch.cuda.synchronize()
+        assert _pool_bytes() == freed
     finally:
         c.close()

@@ -37,8 +37,9 @@ void Context::enter() {
 
 bool give_back_work() {
   Context *C = g_ctx;
-  if (!C || C->work_busy > 0 || !C->crtw) return false;
+  if (!C || C->work_busy > 0 || !(C->crtw || C->gradw)) return false;
   release_crt_work(*C);
+  release_grad_work(*C);
   // the frees are stream-ordered, and the pool keeps what they return
   (void)hipStreamSynchronize(C->stream);
   hipMemPool_t pool = nullptr;

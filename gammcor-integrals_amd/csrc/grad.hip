@@ -33,9 +33,12 @@
 
 namespace gi {
 
-// Device arrays of coulomb_energy_grad, kept in the context and grown only: a
-// program calls it once per geometry, and stream-ordered frees of the slabs at
-// the end of every call cost 16 ms of it after some hundred calls.
+// Device arrays of coulomb_energy_grad, kept in the context and grown only up to
+// GRAD_KEEP bytes: a program calls it once per geometry, and stream-ordered frees
+// of the slabs at the end of every call cost 16 ms of it after some hundred calls
+// of 2 ms.  Beyond that (contracted bases from about 350 AOs on, 60 ms a call)
+// they are freed when the call ends.
+constexpr size_t GRAD_KEEP = 1ull << 30;
 struct GradWork {
   DBuf<double> D, et, rows, dk, part, prow, q;
   DBuf<GradJob> jobs;
@@ -43,6 +46,11 @@ struct GradWork {
   DBuf<int> aoloc, prim0, nprim;
   DBuf<QRec> bra, ket;
   DBuf<CoulKet> kets;
+  size_t bytes() const {
+    return (D.n + et.n + rows.n + dk.n + part.n + prow.n + q.n) * sizeof(double) + jobs.n * sizeof(GradJob) +
+           prim.n * sizeof(PrimRec) + (aoloc.n + prim0.n + nprim.n) * sizeof(int) + (bra.n + ket.n) * sizeof(QRec) +
+           kets.n * sizeof(CoulKet);
+  }
 };
 static GradWork &grad_work(Context &C) {
   if (!C.gradw) C.gradw = new GradWork();
@@ -212,6 +220,14 @@ void coulomb_energy_grad(Context &C, const double *D, long long ldd, double kapp
   if (!C.basis_set) throw Error{4, "basis not set"};
   if (!D || !energy) throw Error{61, "null density or energy pointer"};
   if (ldd < C.nao) throw Error{61, "leading dimension of D smaller than the number of AOs"};
+  struct Busy {   // the arrays are in use until the call ends, by an error too
+    Context &C;
+    explicit Busy(Context &c) : C(c) { ++C.work_busy; }
+    ~Busy() {
+      --C.work_busy;
+      if (C.gradw && C.gradw->bytes() > GRAD_KEEP) release_grad_work(C);
+    }
+  } busy(C);
   const bool want_grad = grad != nullptr;
   const int nsh = C.nshells;
   // shell pairs s0 >= s1, grouped by E = l0 + l1 so that a class is a contiguous range

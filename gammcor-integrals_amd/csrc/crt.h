@@ -21,10 +21,4 @@ bool crt_gemm_nt(Context &C, long long m, long long n, long long k, double alpha
 bool crt_pairs_nt(Context &C, long long m, long long n, long long k, double alpha, const double *X, long long ldx,
                   const int *pq, const double *B, long long ldb, double beta, double *Cd, long long ldc);
 
-// C (m x na nb) = A^T P, A (k x m, lda) column-major, P(g, a + na b) = Xa(g, a) Xb(g, b)
-// (crt_products_pay: whether that is faster than products in memory and a DGEMM)
-bool crt_products_pay(long long m, long long n, long long k);
-bool crt_products_tn(Context &C, long long m, long long na, long long nb, long long k, const double *A, long long lda,
-                     const double *Xa, const double *Xb, long long ldx, double *Cd, long long ldc);
-
 }  // namespace gi

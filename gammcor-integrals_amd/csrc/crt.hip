@@ -9,12 +9,27 @@
 // Scaling.  Row i of A becomes rint(a 2^s_i) with a 2-norm of at most 2^58, the
 // rows of B likewise, so by Cauchy-Schwarz every element of the integer product
 // is below 2^116 in magnitude, and M/2 = 2^116.78 holds it for the fifteen
-// largest such moduli.  An element keeps its whole mantissa unless it is
-// smaller than 2^-5 of its row's norm; the product is then exact up to
-// 2^-58 |a_i| |b_j| from the rounding of small elements, and one rounding at
-// the end.  On the decomposition's own product (Inv_L times V, whose sums
-// cancel by 1e4) that is 2e-13 of the result against 4e-12 for a DGEMM, whose
-// partial sums round at every step; fourteen moduli would lose against it.
+// largest such moduli.  Norms are at least 2^57 and an element is off by half a
+// unit, so an element of the product is off by at most sqrt(k) 2^-57 |a_i| |b_j|
+// (about 2^-59 |a_i| |b_j| in earnest) and one rounding at the end.
+//
+// That is a bound on the rows' norms, where DGEMM's is on the sum of an
+// element's own terms: elements below 2^-5 of their row's norm lose bits, and
+// where the large elements of two rows hardly meet, the small result keeps fewer
+// digits than DGEMM gives it.  So the route serves only products whose operands
+// or whose use have errors of the norms' kind themselves, by far larger ones:
+//   vectors Inv_L V^T: Inv_L is an inverse.  Largest error of the product over
+//     its largest element, 7809 vectors: 1.8e-12, DGEMM 1.2e-11 (its partial sums
+//     cancel by 1e4 and round at every step; fourteen moduli would lose against
+//     it).  Against vectors of an extended-precision factorization (1936, the
+//     scheme modelled) both are off by the same at every magnitude from 1e-3 (a
+//     median of 4.7e-14 of the element, DGEMM 3.1e-14) down to 1e-15 (4.7e-10
+//     and 4.1e-10), where neither has a digit left.
+//   SubtractR M -= L L^T: |L_i|^2 is at most the diagonal integral, the
+//     integrals' own scale; the same pivots.
+//   XR, which a solve with the metric S follows: Z of 1296 points against
+//     extended precision, the same errors at every magnitude (median 3e-8).
+// Products of a caller's own operands (Rkab) stay with DGEMM.
 //
 // Why it pays: fifteen int8 products cost 30 operations per multiply-add, 14 fs
 // at the 2.15 POP/s of the tile kernel (bound by the card's power: it clocks
@@ -93,10 +108,8 @@ static const CrtConst &crt_const_host() {
 }
 
 // ------------------------------------------------------------------ operands
-// element (row, k) of an operand; consecutive rows, or for KMAJOR consecutive k,
-// follow each other in memory
+// element (row, k) of an operand; consecutive rows follow each other in memory
 struct CrtMat {
-  static constexpr bool KMAJOR = false;
   const double *x;
   long long ld;
   __device__ __forceinline__ double at(long long r, long long k) const { return x[r + ld * k]; }
@@ -104,7 +117,6 @@ struct CrtMat {
 // X(g, p) X(g, q) of column k's orbital pair (p, q), halved for p = q, zero for
 // padding columns (p < 0)
 struct CrtPairs {
-  static constexpr bool KMAJOR = false;
   const double *x;
   long long ld;
   const int *pq;
@@ -113,25 +125,6 @@ struct CrtPairs {
     if (p < 0) return 0.0;
     const double v = x[r + ld * p] * x[r + ld * q];
     return p == q ? 0.5 * v : v;
-  }
-};
-
-// rows contiguous in k
-struct CrtRows {
-  static constexpr bool KMAJOR = true;
-  const double *x;
-  long long ld;
-  __device__ __forceinline__ double at(long long r, long long k) const { return x[k + ld * r]; }
-};
-// Xa(k, a) Xb(k, b) of row a + na b
-struct CrtProducts {
-  static constexpr bool KMAJOR = true;
-  const double *xa, *xb;
-  long long ld;
-  unsigned na;
-  __device__ __forceinline__ double at(long long r, long long k) const {
-    const unsigned b = (unsigned)r / na, a = (unsigned)r - b * na;
-    return xa[k + ld * a] * xb[k + ld * b];
   }
 };
 
@@ -153,26 +146,6 @@ __global__ void __launch_bounds__(256) k_crt_sumsq(Src S, long long rows, long l
     nz |= v != 0.0;
   }
   part[blockIdx.y * rows + r] = s == 0.0 && nz ? 4.9406564584124654e-324 : s;
-}
-
-// the same for rows contiguous in k, whole rows: one wave a row
-template <class Src>
-__global__ void __launch_bounds__(256) k_crt_sumsq_rows(Src S, long long rows, long long k0, long long kk, double *part) {
-  const int lane = threadIdx.x & 63;
-  const long long r = blockIdx.x * 4LL + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  if (r >= rows) return;
-  double s = 0.0;
-  bool nz = false;
-#pragma unroll 4
-  for (long long k = lane; k < kk; k += 64) {
-    const double v = S.at(r, k0 + k);
-    s += v * v;
-    nz |= v != 0.0;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  if (lane == 0) part[r] = s;
-  if (s == 0.0 && __ballot(nz) != 0 && lane == 0) part[r] = 4.9406564584124654e-324;
 }
 
 // scale exponents s of the rows: a norm of at most 2^CRT_BITS after scaling;
@@ -210,26 +183,10 @@ __global__ void __launch_bounds__(256) k_crt_residues(Src S, long long r0, long 
   float d[4][16];
   const bool rok = rl < rows;
   const int ex = rok ? e[r0 + rl] : 0;
-  // KMAJOR: the 64 x 64 elements through LDS, a row of 64 k at a time (rows
-  // padded by one against bank conflicts); a lane's own sixteen would touch 64
-  // lines a load
-  __shared__ double tile[Src::KMAJOR ? 64 * 65 : 1];
-  if constexpr (Src::KMAJOR) {
-    const long long k = blockIdx.y * 64LL + lane;
-#pragma unroll 4
-    for (int i = 0; i < 16; ++i) {
-      const int ri = 16 * w + i;
-      const long long r = blockIdx.x * 64LL + ri;
-      tile[ri * 65 + lane] = r < rows && k < kk ? S.at(r0 + r, k0 + k) : 0.0;
-    }
-    __syncthreads();
-  }
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const long long k = 16 * kb + i;
-    double y;
-    if constexpr (Src::KMAJOR) y = tile[lane * 65 + 16 * w + i];
-    else y = rok && k < kk ? S.at(r0 + rl, k0 + k) : 0.0;
+    double y = rok && k < kk ? S.at(r0 + rl, k0 + k) : 0.0;
     y = rint(ldexp(y, ex));
     const double y3 = rint(y * 0x1p-45);
     y = fma(-y3, 0x1p45, y);
@@ -499,32 +456,15 @@ bool crt_pays(long long m, long long n, long long k, double part) {
   return 28.6 * mac > 14.0 * pad + 6500.0 * (double)(m + n) * k + 5000.0 * (double)m * n + 1e11;
 }
 
-// The same for crt_products_tn.  DGEMM takes 34 fs a multiply-add on the shapes
-// of Rkab (51 to 65 TFLOP/s), and as k is short here, the number of points, the
-// ends of the tiles weigh more: 9500 fs a result element.  (H2O)n, 375 n vectors
-// of 225 n^2 pairs at 188 n points, DGEMM and int8: n = 5 442 and 446 us, n = 6
-// 807 and 727 us, n = 8 2.39 and 1.82 ms, n = 12 10.2 and 6.3 ms.  The line lies
-// 400 us higher, what a context's first call pays for the work arrays.
-bool crt_products_pay(long long m, long long n, long long k) {
-  if (m < 512 || n < 512 || k < 512) return false;
-  const double mac = (double)m * n * k, pad = (double)crt_up(m, CRT_T) * crt_up(n, CRT_T) * crt_up(k, CRT_KS);
-  return 34.0 * mac > 14.0 * pad + 6500.0 * (double)(m + n) * k + 9500.0 * (double)m * n + 5e11;
-}
-
-template <class Src>
 static int crt_slices(long long kk) {   // partial sums of a row's squares
-  return Src::KMAJOR ? 1 : (int)((kk + CRT_KSUM - 1) / CRT_KSUM);
+  return (int)((kk + CRT_KSUM - 1) / CRT_KSUM);
 }
 
 template <class Src>
 static void crt_exponents(Context &C, CrtWork &W, const Src &S, long long rows, long long k0, long long kk, int *e) {
-  const int slices = crt_slices<Src>(kk);
-  if constexpr (Src::KMAJOR)
-    hipLaunchKernelGGL(k_crt_sumsq_rows<Src>, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, C.stream, S, rows, k0, kk,
-                       W.part.p);
-  else
-    hipLaunchKernelGGL(k_crt_sumsq<Src>, dim3((unsigned)((rows + 255) / 256), (unsigned)slices), dim3(256), 0, C.stream,
-                       S, rows, k0, kk, W.part.p);
+  const int slices = crt_slices(kk);
+  hipLaunchKernelGGL(k_crt_sumsq<Src>, dim3((unsigned)((rows + 255) / 256), (unsigned)slices), dim3(256), 0, C.stream,
+                     S, rows, k0, kk, W.part.p);
   hipLaunchKernelGGL(k_crt_exps, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, C.stream, W.part.p, rows, slices,
                      e, W.bad.p);
   GI_HIP(hipGetLastError());
@@ -576,7 +516,7 @@ static bool crt_product(Context &C, const SrcA &A, const SrcB &B, long long m, l
     Wp->ea.alloc((size_t)(nkc * mp));
     Wp->eb.alloc((size_t)(nkc * np));
     Wp->bad.alloc(1);
-    Wp->part.alloc((size_t)std::max(crt_slices<SrcA>(kc) * m, crt_slices<SrcB>(kc) * n));
+    Wp->part.alloc((size_t)crt_slices(kc) * std::max(m, n));
     Wp->keep.alloc((size_t)(small * kp / 16 * CRT_N));
     Wp->pass.alloc((size_t)(step * kp / 16 * CRT_N));
     Wp->R.alloc((size_t)(small * step * CRT_N));
@@ -648,12 +588,6 @@ bool crt_gemm_nt(Context &C, long long m, long long n, long long k, double alpha
 bool crt_pairs_nt(Context &C, long long m, long long n, long long k, double alpha, const double *X, long long ldx,
                   const int *pq, const double *B, long long ldb, double beta, double *Cd, long long ldc) {
   return crt_product(C, CrtPairs{X, ldx, pq}, CrtMat{B, ldb}, m, n, k, alpha, beta, Cd, ldc, false);
-}
-
-bool crt_products_tn(Context &C, long long m, long long na, long long nb, long long k, const double *A, long long lda,
-                     const double *Xa, const double *Xb, long long ldx, double *Cd, long long ldc) {
-  if (na * nb >= (1LL << 31)) return false;
-  return crt_product(C, CrtRows{A, lda}, CrtProducts{Xa, Xb, ldx, (unsigned)na}, m, na * nb, k, 1.0, 0.0, Cd, ldc, false);
 }
 
 }  // namespace gi

@@ -512,14 +512,13 @@ void thc_rkab(Context &C, const double *dX, long long ldx, long long npts, const
                          lda_o, &zero, w.Xa.p, npts));
   THC_BLAS(rocblas_dgemm(C.blas, rocblas_operation_none, rocblas_operation_none, npts, NB, nao, &one, dX, ldx, CBo,
                          ldb_o, &zero, w.Xb.p, npts));
-  // Rkab(k, a, b) = sum_g Z(g, k) Xa(g, a) Xb(g, b): on the int8 matrix cores
-  // where that pays, else as DGEMMs, b in chunks of at most 2^26 doubles of
-  // products
-  if (crt_products_pay(nvec, NA * NB, npts) &&
-      crt_products_tn(C, nvec, NA, NB, npts, dZ, ldz, w.Xa.p, w.Xb.p, npts, dRkab, nvec)) {
-    C.wait();
-    return;
-  }
+  // Rkab(k, a, b) = sum_g Z(g, k) Xa(g, a) Xb(g, b), b in chunks of at most
+  // 2^26 doubles of products.  FP64 products only: the operands are the caller's,
+  // and the int8 products (crt.hip) keep an element against its row's norm.  With
+  // orbitals and vectors that decay over 20 bohr an element where the supports
+  // hardly meet was then off by up to 3e-8 of its terms' sum, where DGEMM keeps
+  // 9e-16 (442 us at 5 waters, 2.39 ms at 8, 10.2 ms at 12 against 446 us, 1.82
+  // and 6.3 ms).
   const long long nbc = std::max<long long>(1, std::min<long long>(NB, (1LL << 26) / (npts * NA)));
   w.W.alloc((size_t)(npts * NA * nbc));
   for (long long b = 0; b < NB; b += nbc) {

@@ -121,3 +121,45 @@ def test_work_arrays_are_given_back():
         assert _pool_bytes() == freed
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("work_mb", [9216, 64])   # four chunks of k; some thirty, with slices of vectors
+def test_pair_products_of_orthonormal_points(work_mb):
+    """XR = 2 Xgpq R^T itself: with orthonormal rows of X the metric is the
+    identity (off its diagonal the squares of rounding errors), so Z = XR up to
+    the rounding of S(g, g), some nao units of 2^-52."""
+    b = systems.water_system(11, 8.8, "large", seed=5)
+    c = lib.Context(0)
+    try:
+        c.set_basis(b)
+        c.chol_build(tau=1e-5)
+        c.set_option("int8_work_mb", work_mb)
+        m = c.chol_meta()
+        nv, msd = m["nvecs"], m["max_subset_dim"]
+        n = 768   # three tiles of points: the int8 route is the faster one from some 3500 vectors on
+        assert nv > 3800
+        rng = np.random.default_rng(6)
+        X = np.asfortranarray(np.linalg.qr(rng.standard_normal((b.nao, n)))[0].T)
+        Z, _ = c.thc_z(X)
+        k = np.unique(np.concatenate([[0, 255, 256, nv - 1], rng.choice(nv, 16, replace=False)]))
+        R = torch.as_tensor(_Device(c.chol_rkpq_device_ptr(), (m["nsubsets"], msd, nv)), device="cuda")
+        R = R[:, :, torch.from_numpy(k).cuda()].cpu().numpy()
+    finally:
+        c.close()
+    loc0 = np.concatenate([[0], np.cumsum([b.shell_nang(s) for s in range(b.nshells)])])
+    P, Q, cols = [], [], []
+    for (A, B), (_, pos, sub) in zip(m["shell_pairs"], m["shell_pair_loc"]):
+        na, nb = b.shell_nang(A - 1), b.shell_nang(B - 1)
+        ab = [(i, j) for j in range(nb) for i in range(j if A == B else 0, na)]
+        P += [loc0[A - 1] + i for i, _ in ab]
+        Q += [loc0[B - 1] + j for _, j in ab]
+        cols += [(sub - 1) * msd + pos - 1 + i for i in range(len(ab))]
+    P, Q, V = np.array(P), np.array(Q), R.reshape(-1, len(k))[cols].T
+    g = np.array([0, 1, 255, 256, 257, 511, 512, 700, n - 2, n - 1])
+    A = X[np.ix_(g, P)] * X[np.ix_(g, Q)] * np.where(P == Q, 1.0, 2.0)
+    ref = np.asarray(A, np.longdouble) @ np.asarray(V, np.longdouble).T
+    ref /= (np.asarray(X[g], np.longdouble) ** 2).sum(1)[:, None] ** 2
+    bar = (np.sqrt(len(P)) * 2.0 ** -57 * np.linalg.norm(A, axis=1)[:, None] * np.linalg.norm(V, axis=1)[None, :]
+           + 4 * b.nao * 2.0 ** -52 * np.abs(ref)).astype(float)
+    err = np.abs(Z[np.ix_(g, k)] - ref).astype(float)
+    assert (err <= bar).all(), float((err / bar).max())

@@ -57,6 +57,11 @@ static GradWork &grad_work(Context &C) {
   return *C.gradw;
 }
 void release_grad_work(Context &C) {
+  // the frees follow the context stream; a call that ended by an error may have
+  // left class launches on the side streams that it has not joined
+  if (C.gradw)
+    for (hipStream_t s : C.eri_side)
+      if (s) (void)hipStreamSynchronize(s);
   delete C.gradw;
   C.gradw = nullptr;
 }

@@ -31,13 +31,16 @@
 //     extended precision, the same errors at every magnitude (median 3e-8).
 // Products of a caller's own operands (Rkab) stay with DGEMM.
 //
-// Why it pays: fifteen int8 products cost 30 operations per multiply-add, 14 fs
-// at the 2.15 POP/s of the tile kernel (bound by the card's power: it clocks
-// down to 1.6 GHz), where DGEMM takes 28.6 fs at 70 TFLOP/s.  Norms, conversion
-// and reconstruction move 31 bytes per operand element and up to 38 per result
-// element at memory speed and take back a part (crt_pays).  (H2O)16, 1200 AOs,
-// 7809 vectors of 316,063 pairs: vectors' product 287 -> 165 ms, SubtractR 84 ->
-// 62 ms; XR of 1536 points 115 -> 45 ms.
+// Why it pays: fifteen int8 products cost 30 operations per multiply-add, 12.9 fs
+// on the padded tiles of the vectors' product (2.33 POP/s) and 11 on XR (2.7),
+// where DGEMM takes 28.6 fs at 70 TFLOP/s.  By the cycle counters the clock goes
+// down to 1.6 to 1.77 GHz in those launches (1.44 to 1.76 on XR; 2.4 without such
+// load) and the matrix cores are busy in 64 and 77 % of the cycles.  An operand
+// element moves 31 bytes (read for the norm, read and written as residues), a
+// result element 38 (residues written and read, the result), 46 where it is
+// added to, all at memory speed, which takes back a part (crt_pays).  (H2O)16,
+// 1200 AOs, 7809 vectors of 316,063 pairs: vectors' product 287 -> 165 ms,
+// SubtractR 84 -> 62 ms; XR of 1536 points 115 -> 45 ms.
 //
 // Layout.  Residues of an operand: [modulus][32-row block][32-k block] fragments
 // of 1 KB, lane l of v_mfma_i32_32x32x32_i8 holding row l % 32 and the sixteen k
@@ -311,7 +314,7 @@ __global__ void __launch_bounds__(256, 1) k_crt_gemm(CrtGemm G, const CrtConst *
   for (int q = 0; q < 8; ++q) read(a0, b0, 0, 0, q);
   // One read or copy behind each product: an MFMA holds the matrix core for 32
   // cycles, in which they issue for free; in a group before the products they
-  // left it idle half of the time (1.98 -> 2.38 POP/s).  Scheduling barriers,
+  // left it idle half of the time (1.98 -> 2.38 POP/s when it was made).  Scheduling barriers,
   // since the compiler groups them again.
 #pragma unroll 1
   for (int s = 0; s < nks; ++s) {
@@ -342,7 +345,7 @@ __global__ void __launch_bounds__(256, 1) k_crt_gemm(CrtGemm G, const CrtConst *
   // The quotient's low bits stand in the low bits of x / m + 1.5 2^23, and the
   // byte of x - m q needs no others.  Below 2^22 the float of x is exact and
   // the quotient off from rounding by under 0.001 (the limit is 0.0019: m = 255
-  // must leave |x - m q| <= 128); larger sums, which need a long k, are first
+  // must leave |x - m q| < 128); larger sums, which need a long k, are first
   // brought below 2 m.  Three operations an element, with two integer
   // multiplications and two roundings in their place the ends of the tiles took
   // as long as 18 stages.
@@ -444,12 +447,13 @@ void release_crt_work(Context &C) {
   C.crtw = nullptr;
 }
 
-// The int8 route against DGEMM by their measured rates on one MI355X, in
-// femtoseconds: 28.6 a multiply-add by DGEMM (70 TFLOP/s), 14 in the tile kernel
-// on its padded tiles (2.15 POP/s), 6500 an operand element (norm and
-// conversion, 31 bytes), 5000 a result element (38 bytes with beta), and 100
-// us of launches and the flag's way to the host.  A square product pays from
-// about 1400 on.  `part`: share of the multiply-adds that a triangular A needs.
+// The int8 route against DGEMM on one MI355X, in femtoseconds: 28.6 a
+// multiply-add by DGEMM (70 TFLOP/s), 14 in the tile kernel on its padded tiles
+// (now 11 to 13, see above: the line lies on the safe side), 6500 an operand
+// element (norm and conversion: 6.4 ps measured on XR), 5000 a result element,
+// and 100 us of launches and the flag's way to the host.  By this a square
+// product pays from about 2400 on.  `part`: share of the multiply-adds that a
+// triangular A needs.
 bool crt_pays(long long m, long long n, long long k, double part) {
   if (m < 512 || n < 512 || k < 512) return false;
   const double mac = (double)m * n * k * part, pad = (double)crt_up(m, CRT_T) * crt_up(n, CRT_T) * crt_up(k, CRT_KS) * part;

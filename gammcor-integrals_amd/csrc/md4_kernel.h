@@ -20,10 +20,11 @@
 // Contracted pairs: X accumulates over ket primitives in registers; the
 // block of a contracted bra accumulates over its primitive pairs in place.
 //
-// What bounds it: vector instructions (six or seven per matrix instruction,
-// and FP64 matrix and vector instructions share their units) and the latency
-// of the recursion's levels at two to four waves per SIMD; the matrix
-// instructions take 15 to 30 % of the time, LDS 20 to 45 %.  Sum over the
+// What bounds it: vector instructions (6.2 per matrix instruction over the
+// uncontracted (H2O)16 build, 3.6 to 19 by class, and FP64 matrix and vector
+// instructions share their units) and the latency of the recursion's levels at
+// two to four waves per SIMD; the matrix cores are busy in 15 % of the cycles, 6
+// to 22 % by class, and waves wait in 29 % of theirs.  Sum over the
 // classes, one after the other: (H2O)12, 900 AOs, uncontracted 35.0 -> 30.2 ms,
 // (H2O)5, 375 AOs, contracted 216 -> 135 ms, from the recursion by levels at
 // LDS latency (md4_rtable), Boys passes over several primitive steps, and

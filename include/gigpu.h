@@ -59,9 +59,11 @@ typedef struct gi_context gi_context;
 /* Create a context on HIP device `device` (no reference counterpart: the
  * reference initialises module state in chol_gammcor_Rkpq,
  * Cholesky_Gammcor.f90:347-352).  A context keeps its device work arrays
- * (the Cholesky panels, the vector staging, the factorization scratch and
- * the split-product slices) across calls, grown only, so that repeated
- * builds allocate nothing; gi_destroy frees them. */
+ * (the Cholesky panels, the vector staging, the factorization scratch, the
+ * split-product slices, the arrays of the int8 products within int8_work_mb,
+ * up to 1 GiB of the Coulomb gradient) across calls, grown only, so that
+ * repeated builds allocate nothing; gi_destroy frees them, and those of the
+ * int8 products and the gradient go when another allocation fails. */
 int gi_create(gi_context **ctx, int64_t device);
 int gi_destroy(gi_context *ctx);
 /* Message of the last failure on this thread (replaces msg(...,MSG_ERROR) +
